@@ -6,9 +6,10 @@
 // Q4_0 and Q8_0 are one exact-integer-times-scale product each; Q6_K is
 // (d*sc)*q, two roundings in that order (q6_k.rs:41-44).
 //
-// Work split: one thread writes 8 consecutive outputs, so consecutive
-// threads store consecutive 32-byte runs (coalesced); the few block bytes
-// each thread needs are re-read by its neighbours from L1.
+// Work split of a 16-byte aligned output (dequant_rows_kernel): a lane makes
+// 16 bytes of output per store, so every store instruction of a wave writes
+// 1 KB of consecutive bytes.  Unaligned outputs take one thread per 8 outputs
+// with element stores.
 #include "swamp_common.hpp"
 
 namespace {
@@ -21,42 +22,16 @@ __device__ __forceinline__ uint32_t ld_u16(const uint8_t *p) {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
-template <bool kVec>
-__device__ __forceinline__ void store8(float *dst, size_t base, size_t n,
-                                       const float (&v)[8]) {
-  if (kVec && base + 8 <= n) {
-    float4 *p = reinterpret_cast<float4 *>(dst + base);
-    p[0] = make_float4(v[0], v[1], v[2], v[3]);
-    p[1] = make_float4(v[4], v[5], v[6], v[7]);
-  } else {
+__device__ __forceinline__ void store8(float *dst, size_t base, size_t n, const float (&v)[8]) {
 #pragma unroll
-    for (int j = 0; j < 8; j++)
-      if (base + j < n) dst[base + j] = v[j];
-  }
-}
-
-// bf16 output (the dequant-once GEMM route): each exact fp32 value rounded
-// to nearest even, as the fused GEMM rounds its in-register weights.
-template <bool kVec>
-__device__ __forceinline__ void store8(__bf16 *dst, size_t base, size_t n,
-                                       const float (&v)[8]) {
-  if (kVec && base + 8 <= n) {
-    bf16x8_t b;
-#pragma unroll
-    for (int j = 0; j < 8; j++) b[j] = __bf16(v[j]);
-    *reinterpret_cast<bf16x8_t *>(dst + base) = b;
-  } else {
-#pragma unroll
-    for (int j = 0; j < 8; j++)
-      if (base + j < n) dst[base + j] = __bf16(v[j]);
-  }
+  for (int j = 0; j < 8; j++)
+    if (base + j < n) dst[base + j] = v[j];
 }
 
 // q4_0::dequant (q4_0.rs:22-37): element i of a block is byte i/2, low
 // nibble for even i; value (nib - 8) * f16(d).
-template <bool kVec, class T = float>
 __global__ void dequant_q4_0_kernel(const uint8_t *__restrict__ raw,
-                                    T *__restrict__ dst, size_t n) {
+                                    float *__restrict__ dst, size_t n) {
   const size_t g = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const size_t base = g * 8;
   if (base >= n) return;
@@ -71,13 +46,12 @@ __global__ void dequant_q4_0_kernel(const uint8_t *__restrict__ raw,
     const int q = int((nib >> (4 * j)) & 0xFu);  // byte j/2, low nibble first
     v[j] = float(q - 8) * d;
   }
-  store8<kVec>(dst, base, n, v);
+  store8(dst, base, n, v);
 }
 
 // q8_0::dequant scalar arm (q8_0.rs:127-139): value int8 * f16(d).
-template <bool kVec, class T = float>
 __global__ void dequant_q8_0_kernel(const uint8_t *__restrict__ raw,
-                                    T *__restrict__ dst, size_t n) {
+                                    float *__restrict__ dst, size_t n) {
   const size_t g = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const size_t base = g * 8;
   if (base >= n) return;
@@ -94,15 +68,14 @@ __global__ void dequant_q8_0_kernel(const uint8_t *__restrict__ raw,
     v[j] = float(int8_t(uint8_t(lo >> (8 * j)))) * d;
     v[4 + j] = float(int8_t(uint8_t(hi >> (8 * j)))) * d;
   }
-  store8<kVec>(dst, base, n, v);
+  store8(dst, base, n, v);
 }
 
 // q4_k::dequant_scalar (q4_k.rs:278-321) with unpack_scales (:37-53),
 // layout A: pair p = sub-blocks (2p, 2p+1) use qs[32p..32p+32], low nibble
 // for the even sub-block, high nibble for the odd one.
-template <bool kVec, class T = float>
 __global__ void dequant_q4_k_kernel(const uint8_t *__restrict__ raw,
-                                    T *__restrict__ dst, size_t n) {
+                                    float *__restrict__ dst, size_t n) {
   const size_t g = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const size_t base = g * 8;
   if (base >= n) return;
@@ -141,7 +114,7 @@ __global__ void dequant_q4_k_kernel(const uint8_t *__restrict__ raw,
     const float t = sv * float(qi);
     v[j] = t - mv;
   }
-  store8<kVec>(dst, base, n, v);
+  store8(dst, base, n, v);
 }
 
 // q6_k::dequant_scalar (q6_k.rs:22-56): the 8 outputs of a thread are
@@ -150,9 +123,8 @@ __global__ void dequant_q4_k_kernel(const uint8_t *__restrict__ raw,
 // (low for j < 2, high for j >= 2), bits 4-5 are bits 2j..2j+1 of
 // qh[32h + l], and all 8 share the int8 scale sc[8h + l0/16 + 2j]; value
 // (d * sc) * (q - 32).  Blocks are 210 bytes, so only 2-byte loads.
-template <bool kVec, class T = float>
 __global__ void dequant_q6_k_kernel(const uint8_t *__restrict__ raw,
-                                    T *__restrict__ dst, size_t n) {
+                                    float *__restrict__ dst, size_t n) {
   const size_t g = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const size_t base = g * 8;
   if (base >= n) return;
@@ -178,7 +150,127 @@ __global__ void dequant_q6_k_kernel(const uint8_t *__restrict__ raw,
     const int q = int(((lb >> nsh) & 0xFu) | (((hb >> (2 * j)) & 3u) << 4)) - 32;
     v[k] = ds * float(q);
   }
-  store8<kVec>(dst, base, n, v);
+  store8(dst, base, n, v);
+}
+
+// ---- 16-byte aligned output -------------------------------------------------
+// Bound by the output's bytes (4 or 2 per weight against 0.56-1.06 read).  A
+// lane makes 16 consecutive bytes (E weights: 4 fp32, 8 bf16) per step and a
+// wave two steps of 1 KB, whose loads are all issued before the first
+// conversion.  Stores of fp32 are non-temporal: the output is larger than
+// the caches' share and is not read back here.  14336 x 4096 weights, us (one
+// thread per 8 outputs, two 16-byte stores 32 bytes apart / this kernel):
+// fp32 Q4_0 43.4 / 37.4, Q8_0 65.5 / 41.7, Q4_K 44.9 / 37.7, Q6_K 64.5 / 40.1
+// (7.05-7.17 TB/s); bf16 Q6_K 29.7 / 25.4.  One step per wave measured 39-62
+// us, four 38-43; temporal stores 38.5-54.
+// Values are those of the kernels above: V_CVT_F32_F16 gives the bits of
+// f16_bits_to_f32_exact for all 65536 halves, NaN payloads included.
+constexpr int kSteps = 2;
+
+template <int DT, class T>
+__global__ void __launch_bounds__(256) dequant_rows_kernel(const uint8_t *__restrict__ raw,
+                                                           T *__restrict__ dst, size_t n) {
+  constexpr int E = 16 / int(sizeof(T));
+  constexpr int kBlk = DT == SWAMP_Q4_0 || DT == SWAMP_Q8_0 ? 32 : 256;
+  constexpr int kBytes =
+      DT == SWAMP_Q4_0 ? 18 : DT == SWAMP_Q8_0 ? 34 : DT == SWAMP_Q4_K ? 144 : 210;
+  static_assert(E == 4 || DT == SWAMP_Q6_K, "bf16 output of the other formats: kernels below");
+  const size_t wave =
+      size_t(blockIdx.x) * 4 + size_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+  const size_t first = wave * (kSteps * 64 * E) + size_t(threadIdx.x & 63) * E;
+  uint32_t q[kSteps][E / 4];                   // 4 codes (Q4_0: their 2 bytes) each
+  [[maybe_unused]] uint32_t qh[kSteps][E / 4];  // Q6_K high bits
+  uint32_t hd[kSteps][4];                      // scales
+#pragma unroll
+  for (int u = 0; u < kSteps; u++) {
+    const size_t base = first + size_t(u) * 64 * E;
+    const size_t bs = base < n ? base : 0;  // past the end: re-read the first block
+    const int e0 = int(bs % kBlk);
+    const uint8_t *blk = raw + bs / kBlk * kBytes;
+    if constexpr (DT == SWAMP_Q4_0) {
+      q[u][0] = ld_u16(blk + 2 + e0 / 2);
+      hd[u][0] = ld_u16(blk);
+    } else if constexpr (DT == SWAMP_Q8_0) {
+      q[u][0] = ld_u16(blk + 2 + e0) | ld_u16(blk + 4 + e0) << 16;
+      hd[u][0] = ld_u16(blk);
+    } else if constexpr (DT == SWAMP_Q4_K) {
+      const uint4 h = *reinterpret_cast<const uint4 *>(blk);
+      hd[u][0] = h.x;
+      hd[u][1] = h.y;
+      hd[u][2] = h.z;
+      hd[u][3] = h.w;
+      q[u][0] = *reinterpret_cast<const uint32_t *>(blk + 16 + 32 * (e0 >> 6) + (e0 & 31));
+    } else {
+      const int h = e0 >> 7, j = (e0 >> 5) & 3, l0 = e0 & 31;
+      const uint8_t *ql = blk + 64 * h + 32 * (j & 1) + l0, *hb = blk + 128 + 32 * h + l0;
+#pragma unroll
+      for (int k = 0; k < E / 4; k++) {
+        q[u][k] = ld_u16(ql + 4 * k) | ld_u16(ql + 4 * k + 2) << 16;
+        qh[u][k] = ld_u16(hb + 4 * k) | ld_u16(hb + 4 * k + 2) << 16;
+      }
+      hd[u][0] = ld_u16(blk + 208);
+      hd[u][1] = blk[192 + 8 * h + (l0 >> 4) + 2 * j];
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kSteps; u++) {
+    const size_t base = first + size_t(u) * 64 * E;
+    if (base >= n) return;
+    const int e0 = int(base % kBlk);
+    const float d = swamp::f16_bits_to_f32(hd[u][0]);
+    float v[E];
+    if constexpr (DT == SWAMP_Q4_0) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[k] = float(int((q[u][0] >> (4 * k)) & 0xFu) - 8) * d;
+    } else if constexpr (DT == SWAMP_Q8_0) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[k] = float(int8_t(uint8_t(q[u][0] >> (8 * k)))) * d;
+    } else if constexpr (DT == SWAMP_Q4_K) {
+      const int sb = e0 >> 5;
+      const uint32_t sh = 8u * uint32_t(sb & 3);
+      const uint32_t s03 = hd[u][1] >> sh, s47 = hd[u][2] >> sh, s811 = hd[u][3] >> sh;
+      const uint32_t scale = sb < 4 ? s03 & 63u : (s811 & 0xFu) | ((s03 >> 2) & 0x30u);
+      const uint32_t mn = sb < 4 ? s47 & 63u : ((s811 >> 4) & 0xFu) | ((s47 >> 2) & 0x30u);
+      const float sv = d * float(scale);
+      const float mv = swamp::f16_bits_to_f32(hd[u][0] >> 16) * float(mn);
+      const uint32_t w = (q[u][0] >> (sb & 1 ? 4 : 0)) & 0x0F0F0F0Fu;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const float t = sv * float((w >> (8 * k)) & 0xFFu);
+        v[k] = t - mv;
+      }
+    } else {
+      const int j = (e0 >> 5) & 3;
+      const float ds = d * float(int8_t(uint8_t(hd[u][1])));
+#pragma unroll
+      for (int k = 0; k < E / 4; k++) {
+        const uint32_t w = ((q[u][k] >> (j & 2 ? 4 : 0)) & 0x0F0F0F0Fu) |
+                           (((qh[u][k] >> (2 * j)) & 0x03030303u) << 4);
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[4 * k + i] = ds * float(int((w >> (8 * i)) & 0xFFu) - 32);
+      }
+    }
+    if (base + E > n) {  // the last lane of an n that is no multiple of E
+#pragma unroll
+      for (int k = 0; k < E; k++)
+        if (base + k < n) dst[base + k] = T(v[k]);
+    } else if constexpr (E == 4) {
+      typedef float f32x4_t __attribute__((ext_vector_type(4)));
+      __builtin_nontemporal_store(f32x4_t{v[0], v[1], v[2], v[3]},
+                                  reinterpret_cast<f32x4_t *>(dst + base));
+    } else {
+      bf16x8_t b;
+#pragma unroll
+      for (int k = 0; k < E; k++) b[k] = __bf16(v[k]);
+      *reinterpret_cast<bf16x8_t *>(dst + base) = b;
+    }
+  }
+}
+
+template <int DT, class T>
+void launch_rows(const uint8_t *raw, T *dst, size_t n, hipStream_t s) {
+  constexpr size_t per = 256 * (16 / sizeof(T)) * kSteps;  // weights per workgroup
+  dequant_rows_kernel<DT, T><<<unsigned((n + per - 1) / per), 256, 0, s>>>(raw, dst, n);
 }
 
 __global__ void dequant_f16_kernel(const uint16_t *__restrict__ raw,
@@ -206,20 +298,20 @@ int swamp_launch_dequant(uint32_t dtype, const void *d_raw, float *d_dst,
   const dim3 grid1(unsigned((n + threads - 1) / threads));
   switch (dtype) {
   case SWAMP_Q4_0:
-    if (vec) dequant_q4_0_kernel<true><<<grid8, threads, 0, s>>>(raw, d_dst, n);
-    else dequant_q4_0_kernel<false><<<grid8, threads, 0, s>>>(raw, d_dst, n);
+    if (vec) launch_rows<SWAMP_Q4_0>(raw, d_dst, n, s);
+    else dequant_q4_0_kernel<<<grid8, threads, 0, s>>>(raw, d_dst, n);
     break;
   case SWAMP_Q8_0:
-    if (vec) dequant_q8_0_kernel<true><<<grid8, threads, 0, s>>>(raw, d_dst, n);
-    else dequant_q8_0_kernel<false><<<grid8, threads, 0, s>>>(raw, d_dst, n);
+    if (vec) launch_rows<SWAMP_Q8_0>(raw, d_dst, n, s);
+    else dequant_q8_0_kernel<<<grid8, threads, 0, s>>>(raw, d_dst, n);
     break;
   case SWAMP_Q4_K:
-    if (vec) dequant_q4_k_kernel<true><<<grid8, threads, 0, s>>>(raw, d_dst, n);
-    else dequant_q4_k_kernel<false><<<grid8, threads, 0, s>>>(raw, d_dst, n);
+    if (vec) launch_rows<SWAMP_Q4_K>(raw, d_dst, n, s);
+    else dequant_q4_k_kernel<<<grid8, threads, 0, s>>>(raw, d_dst, n);
     break;
   case SWAMP_Q6_K:
-    if (vec) dequant_q6_k_kernel<true><<<grid8, threads, 0, s>>>(raw, d_dst, n);
-    else dequant_q6_k_kernel<false><<<grid8, threads, 0, s>>>(raw, d_dst, n);
+    if (vec) launch_rows<SWAMP_Q6_K>(raw, d_dst, n, s);
+    else dequant_q6_k_kernel<<<grid8, threads, 0, s>>>(raw, d_dst, n);
     break;
   case SWAMP_F16:
     dequant_f16_kernel<<<grid1, threads, 0, s>>>(static_cast<const uint16_t *>(d_raw), d_dst, n);
@@ -386,13 +478,11 @@ int swamp_launch_dequant_bf16(uint32_t dtype, const void *d_raw, void *d_dst, si
     if (n % 256 != 0) return SWAMP_EINVAL;
     q4k_to_bf16_kernel<<<grid, 256, 0, s>>>(raw, dst, units);
     break;
-  case SWAMP_Q6_K: {
-    // 210-byte blocks, 2-byte aligned: the 8-outputs-per-thread kernel
+  case SWAMP_Q6_K:
+    // 210-byte blocks, 2-byte aligned: the lane-contiguous kernel
     if (n % 256 != 0) return SWAMP_EINVAL;
-    const dim3 grid8(unsigned(((n + 7) / 8 + 255) / 256));
-    dequant_q6_k_kernel<true, __bf16><<<grid8, 256, 0, s>>>(raw, dst, n);
+    launch_rows<SWAMP_Q6_K>(raw, dst, n, s);
     break;
-  }
   default:
     return SWAMP_EDTYPE;
   }
