@@ -742,13 +742,41 @@ __device__ __forceinline__ void stage_vec(uint8_t *lds, const float *v, int ipr,
   }
 }
 
+// silu(gate) * up of a vector of ipr items into lds, in stage_vec's layout:
+// wave w makes units [64 k, 64 k + 64) for k = w, w + kWaves, ..., kN of
+// them.  Loaded through registers, so that one region holds the product: with
+// gate and up both in LDS (2 x 64 KB for rows of up to 16384 weights) a CU
+// held one workgroup of the down projection, and the 8 waves per CU its grid
+// aims for ran as two rounds of 4.
+template <int DT, int kWaves, int kN>
+struct Product {
+  float4 g[kN], u[kN];
+  __device__ __forceinline__ void load(const float *gate, const float *up, int ipr, int wave,
+                                       int lane) {
+    const __amdgpu_buffer_rsrc_t rg = swamp::make_rsrc(gate, uint32_t(ipr) * 256u);
+    const __amdgpu_buffer_rsrc_t ru = swamp::make_rsrc(up, uint32_t(ipr) * 256u);
+#pragma unroll
+    for (int k = 0; k < kN; k++) {
+      const int unit = 64 * (wave + k * kWaves) + lane, it = unit >> 4;
+      const uint32_t off = x_chunk_bytes<DT>(it, (unit & 15) ^ (it & 15));  // past the end: zeros
+      g[k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rg, off, 0, 0));
+      u[k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(ru, off, 0, 0));
+    }
+  }
+  __device__ __forceinline__ void store(uint8_t *lds, int wave, int lane) const {
+#pragma unroll
+    for (int k = 0; k < kN; k++)
+      *reinterpret_cast<float4 *>(lds + 16 * (64 * (wave + k * kWaves) + lane)) = make_float4(
+          swamp::silu_mul(g[k].x, u[k].x), swamp::silu_mul(g[k].y, u[k].y),
+          swamp::silu_mul(g[k].z, u[k].z), swamp::silu_mul(g[k].w, u[k].w));
+  }
+};
+
 __device__ __forceinline__ void read_vec(float4 (&xv)[16], const uint8_t *lds, int item) {
 #pragma unroll
   for (int c = 0; c < 16; c++)
     xv[c] = *reinterpret_cast<const float4 *>(lds + 16 * (16 * item + (c ^ (item & 15))));
 }
-
-using swamp::silu_mul;
 
 // One row set = 64 * kWaves lanes; lane j owns items j, j + T, ... (kPPT
 // items per lane), covering one row of ipr items.  A workgroup is kSets row
@@ -808,7 +836,9 @@ __global__ void __launch_bounds__(64 * kWaves * kSets)
     ya = t0.y[store_row<kRows, kWaves>(t0, tid)];
   }
   constexpr bool kStage = kPPT == 1;  // x through LDS (item count <= 64 kWaves)
-  constexpr bool kTwo = kStage && kPro != kProNone && kWaves <= 4;  // both vectors at once
+  constexpr bool kSwi = kPro == kProSwiGLU || kPro == kProSwiGLUAcc;
+  static_assert(kStage || !kSwi, "SwiGLU: one item per lane");
+  constexpr bool kTwo = kStage && kPro == kProRmsNorm && kWaves <= 4;  // both vectors at once
   constexpr int kRegion = kWaves * 16384;
   __shared__ __align__(16) uint8_t xlds[kStage ? (kTwo ? 2 : 1) * kRegion : 16];
   // waves of the workgroup and this wave's index among them (x staging)
@@ -816,7 +846,10 @@ __global__ void __launch_bounds__(64 * kWaves * kSets)
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)), lane = tid & 63;
   float4 x4[kPPT][16];
   [[maybe_unused]] float4 v4[kPPT][16];  // prologue operand (w_norm or up)
-  if constexpr (kStage) {
+  [[maybe_unused]] Product<DT, kWgWaves, kSwi ? 16 / kSets : 1> prod;
+  if constexpr (kSwi) {
+    prod.load(x, pro.x2, ipr, wave, lane);
+  } else if constexpr (kStage) {
     stage_vec<DT, kWgWaves>(xlds, x, ipr, wave, lane);
     if constexpr (kTwo) stage_vec<DT, kWgWaves>(xlds + kRegion, pro.x2, ipr, wave, lane);
   } else {
@@ -833,7 +866,12 @@ __global__ void __launch_bounds__(64 * kWaves * kSets)
   // keep every load of the tile ahead of the arithmetic (the scheduler would
   // otherwise sink them into registers freed by the current tile)
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (kStage) {
+  if constexpr (kSwi) {
+    prod.store(xlds, wave, lane);  // waits for gate and up, not for the tile
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    st.mark(1);
+    read_vec(x4[0], xlds, item[0]);
+  } else if constexpr (kStage) {
     // the memory counter is in order: waiting until only the tile's loads
     // are outstanding means every DMA of this wave has landed; the barrier
     // covers the other waves' pieces.  Exactly these loads follow the DMA
@@ -851,17 +889,6 @@ __global__ void __launch_bounds__(64 * kWaves * kSets)
       asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
       read_vec(v4[0], xlds, item[0]);
     }
-  }
-  if constexpr (kPro == kProSwiGLU || kPro == kProSwiGLUAcc) {
-#pragma unroll
-    for (int j = 0; j < kPPT; j++)
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        float4 &g = x4[j][i];
-        const float4 u = v4[j][i];
-        g = make_float4(silu_mul(g.x, u.x), silu_mul(g.y, u.y), silu_mul(g.z, u.z),
-                        silu_mul(g.w, u.w));
-      }
   }
   // RMSNorm: W ((x * inv_rms) * w) = inv_rms * (W (x * w)), so the fragment
   // is built from x * w at once, the sum of squares finishes behind it and
