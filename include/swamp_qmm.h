@@ -222,14 +222,16 @@ SWAMP_API int swamp_qgemv_batched(uint32_t dtype, const void *d_w, size_t w_len,
  * bf16 (every tile reads the quantized blocks: 0.56-1.06 bytes per
  * weight); when the tiles do not fill the GPU, K is split across
  * workgroups whose partial tiles go to scratch and are summed in piece
- * order by a second kernel (deterministic).  For Q6_K at any length, and
+ * order by a second kernel (deterministic).  For Q6_K of at most 64 tokens,
+ * of rows of an odd number of blocks, or of many tokens (more than 512, when
+ * the rows are short or the tiles fill the GPU), and otherwise
  * from 1024 tokens when 256 x 256 tiles would fill more than half but not
  * all of the CUs (e.g. 2048 tokens x 6144 rows), the weights are instead
  * dequantized once per call to bf16 in scratch (row chunks of at most
  * 512 MB; the same bf16 values) and each chunk runs through this library's
  * plain bf16 x bf16 -> fp32 MFMA GEMM, whose 192- and 128-row tiles fill
- * the CUs; when that scratch cannot be had the fused kernel runs (Q6_K:
- * SWAMP_EWORKSPACE).  Both routes sum in a fixed order: repeated calls
+ * the CUs; when that scratch cannot be had the fused kernel runs (Q6_K, also
+ * for the partial tiles of its fused kernel: SWAMP_EWORKSPACE).  Both routes sum in a fixed order: repeated calls
  * give the same bits. */
 SWAMP_API int swamp_qgemm(uint32_t dtype, const void *d_w, size_t w_len,
                 const void *d_x, uint32_t x_type, float *d_y, int m,
