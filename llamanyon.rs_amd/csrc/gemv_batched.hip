@@ -678,6 +678,144 @@ __global__ void __launch_bounds__(kThreads, 1) gemv_batched_kernel(Args a) {
   }
 }
 
+// ---- few tokens: x straight from memory to registers -------------------------
+// A decode layer's projections at a handful of tokens move so few weights that
+// staging all of x through LDS behind a barrier, or the second kernel that sums
+// the K groups, bounds the kernel above.  Here a wave's share of x never leaves
+// its registers: one workgroup owns nt <= kT tiles; of every K pass wave w takes
+// quad w (4 items, 256 weights), loads its tokens' x there as fp32, rounds it to
+// the same fp16 fragments and multiplies every tile's quad by them.  The partial
+// tiles meet once, in LDS, summed in wave order (deterministic).
+//  * kT == 1 (at most 16 x the CUs rows): 16 waves, so that a row of up to 4096
+//    weights is a single pass, whose x and weights are all in flight at once.
+//  * kT > 1: 8 waves with room to prefetch: x one pass ahead, weights 2 or 4
+//    units (a tile's quad) ahead.
+template <int kT>
+constexpr int xs_waves() { return kT == 1 ? 16 : 8; }
+
+template <int DT, int kT>
+__global__ void __launch_bounds__(64 * xs_waves<kT>()) gemv_xs_kernel(Args a, int nt) {
+  constexpr int kXsWaves = xs_waves<kT>();
+  __shared__ float part[kXsWaves][kT][256];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const uint32_t rb = a.row_bytes;
+  const uint32_t lane_off = uint32_t(r16) * rb + lane_item_offset<DT>(g);
+  const int n_tiles = (a.n_rows + kRowsTile - 1) / kRowsTile;
+  const int tile0 = int(blockIdx.x) * nt;
+  const int nq = a.ipr / 4, passes = (nq + kXsWaves - 1) / kXsWaves;
+  // x: a lane past the last token starts past the descriptor and reads zeros
+  const uint32_t xbytes = uint32_t(a.n_tok) * uint32_t(a.n_cols) * 4u;
+  const uint32_t xlane = uint32_t(r16) * uint32_t(a.n_cols) * 4u + 4u * uint32_t(x_item_base<DT>(g));
+
+  auto load_xq = [&](float4 (&v)[16], int p) {
+    const int q = p * kXsWaves + wave;
+    const uint32_t so = q < nq ? uint32_t(q) * 1024u : 0u;
+    const __amdgpu_buffer_rsrc_t rs = swamp::make_rsrc(a.x, q < nq ? xbytes : 0u);
+#pragma unroll
+    for (int st = 0; st < 8; st++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        v[2 * st + h] = __builtin_bit_cast(
+            float4, __builtin_amdgcn_raw_buffer_load_b128(
+                        rs, xlane + 4u * uint32_t(stage_elem<DT>(st, 4 * h)), so, 0));
+  };
+  auto to_frags = [&](half8_t (&f)[8], const float4 (&v)[16]) {
+#pragma unroll
+    for (int st = 0; st < 8; st++) {
+      const float e[8] = {v[2 * st].x,     v[2 * st].y,     v[2 * st].z,     v[2 * st].w,
+                          v[2 * st + 1].x, v[2 * st + 1].y, v[2 * st + 1].z, v[2 * st + 1].w};
+#pragma unroll
+      for (int i = 0; i < 8; i++) f[st][i] = _Float16(e[slot_local<DT>(i)]);
+    }
+  };
+  auto load_w = [&](Raw<DT> &r, int p, int t) {
+    const int q = p * kXsWaves + wave, tile = tile0 + t;
+    const uint32_t qs = q < nq ? uint32_t(q) : 0u;
+    const int row0 = min(tile, n_tiles - 1) * kRowsTile;
+    const int nr = q < nq && tile < n_tiles ? min(kRowsTile, a.n_rows - row0) : 0;
+    const __amdgpu_buffer_rsrc_t rs = swamp::make_rsrc(a.w + size_t(row0) * rb, uint32_t(nr) * rb);
+    if constexpr (DT == SWAMP_Q6_K)
+      swamp::load_raw_buf<DT>(r, rs, lane_off, (qs * 210u) & ~3u, g);
+    else
+      load_item<DT>(r, rs, lane_off, qs * quad_bytes<DT>(), g);
+  };
+
+  float4_t acc[kT];
+#pragma unroll
+  for (int t = 0; t < kT; t++) acc[t] = float4_t{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](const Raw<DT> &r, const half8_t (&f)[8], int p, float4_t &c) {
+    Q4kScales kq{};
+    if constexpr (DT == SWAMP_Q4_K) kq = q4k_item_scales(r, g);
+    Q6kScales q6{};
+    [[maybe_unused]] const uint32_t sh6 = 2u * uint32_t((p * kXsWaves + wave) & 1);
+    if constexpr (DT == SWAMP_Q6_K) q6 = q6k_item_scales(r, g, sh6);
+#pragma unroll
+    for (int st = 0; st < 8; st++) {
+      half8_t wb;
+      if constexpr (DT == SWAMP_Q6_K) wb = weights_step_q6k(r, q6, sh6, st);
+      else wb = weights_step<DT>(r, st, kq);
+      c = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[st], wb, c, 0, 0, 0);
+    }
+  };
+
+  if constexpr (kT == 1) {
+    // 16 waves: rows of at most 4096 weights are one pass
+    for (int p = 0; p < passes; p++) {
+      float4 xv[16];
+      half8_t xf[8];
+      Raw<DT> w;
+      load_xq(xv, p);
+      load_w(w, p, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      to_frags(xf, xv);
+      multiply(w, xf, p, acc[0]);
+    }
+  } else {
+    // Units of weights (a pass's tiles, then the next pass's) are issued
+    // kAhead units before they are multiplied, x one pass before.  kAhead
+    // divides kT: unit t's buffer is w[t % kAhead] in every pass.
+    constexpr int kAhead = kT >= 4 && (DT == SWAMP_Q4_0 || DT == SWAMP_Q4_K) ? 4 : 2;
+    float4 xv[16];
+    half8_t xf[8];
+    Raw<DT> w[kAhead];
+    auto load_unit = [&](Raw<DT> &r, int p, int t) {  // t: a constant below 2 kT
+      const int tt = t % kT;
+      load_w(r, p + t / kT, tt < nt ? tt : n_tiles);
+    };
+    load_xq(xv, 0);
+#pragma unroll
+    for (int t = 0; t < kAhead; t++) load_unit(w[t], 0, t);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int p = 0; p < passes; p++) {
+      to_frags(xf, xv);
+      load_xq(xv, p + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < kT; t++) {
+        multiply(w[t % kAhead], xf, p, acc[t]);
+        load_unit(w[t % kAhead], p, t + kAhead);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < kT; t++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) part[wave][t][(4 * g + i) * 16 + r16] = acc[t][i];
+  __syncthreads();
+  const Out out{a.y, a.accumulate};
+  for (int o = tid; o < nt * 256; o += 64 * kXsWaves) {
+    const int t = o >> 8, e = o & 255;
+    if (tile0 + t >= n_tiles) break;
+    float sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < kXsWaves; w++) sum += part[w][t][e];
+    put_y(a, out, e >> 4, (tile0 + t) * kRowsTile + (e & 15), sum);
+  }
+}
+
 // Sum of the K groups' partials, in K-group order (deterministic):
 // y = sum, or y += sum with accumulate.  Up to 16 partials are loaded
 // before any is added, so their latencies overlap.
@@ -747,6 +885,45 @@ int launch_geo(Args a, int lwk, int nkg, hipStream_t s) {
     if (hipGetLastError() != hipSuccess) return SWAMP_ELAUNCH;
   }
   return SWAMP_OK;
+}
+
+template <int DT, int kT>
+int launch_xs_t(const Args &a, int nt, hipStream_t s) {
+  const int n_tiles = (a.n_rows + kRowsTile - 1) / kRowsTile;
+  gemv_xs_kernel<DT, kT><<<unsigned((n_tiles + nt - 1) / nt), 64 * xs_waves<kT>(), 0, s>>>(a, nt);
+  return hipGetLastError() == hipSuccess ? SWAMP_OK : SWAMP_ELAUNCH;
+}
+template <int DT>
+int launch_xs(const Args &a, hipStream_t s) {
+  const int n_tiles = (a.n_rows + kRowsTile - 1) / kRowsTile;
+  const int cus = swamp::device_info().num_cus;
+  const int nt = std::min(8, (n_tiles + cus - 1) / cus);
+  if (nt == 1) return launch_xs_t<DT, 1>(a, nt, s);
+  if (nt == 2) return launch_xs_t<DT, 2>(a, nt, s);
+  if (nt <= 4) return launch_xs_t<DT, 4>(a, nt, s);
+  return launch_xs_t<DT, 8>(a, nt, s);
+}
+// Passes for gemv_xs_kernel: x read once per workgroup, so few tokens times a
+// short row, and tiles for at most one round of workgroups.  us, the kernel
+// above / gemv_xs: Q4_K 4096 x 4096 at 3, 5, 8 tokens 7.2 / 6.4, 9.6 / 7.0,
+// 9.6 / 9.4, at 12 9.7 / 13.4; Q6_K 1024 x 4096 at 5 10.6 / 7.7; Q8_0
+// 4096 x 3072 at 5 8.5 / 6.7; rows of 14336 weights 14.5 / 22.0.  More rows
+// than 4096 take 2 to 8 tiles per workgroup, whose 8 waves are all busy when
+// the row is whole 2048-weight passes: Q4_K 14336 x 4096 at 5 14.8 / 13.2,
+// 9000 x 3072 10.5 / 10.6, 28672 x 4096 at 8 21.1 / 21.6; Q8_0 28672 x 4096 at
+// 5 and 16 32.8 / 31.1, 36.6 / 35.5; 128256 x 4096 at 5 108 / 120.
+bool xs_route(uint32_t dtype, int n_tok, int n_rows, int n_cols) {
+  const int n_tiles = (n_rows + kRowsTile - 1) / kRowsTile;
+  const int cus = swamp::device_info().num_cus;
+  const int nt = (n_tiles + cus - 1) / cus;  // tiles per workgroup
+  const long nx = long(n_tok) * n_cols;
+  if (n_tok > 16 || n_cols % 256 != 0) return false;
+  if (nt <= 1) return n_cols <= 4096 && nx <= 32768;
+  if (n_cols % 2048 != 0) return false;
+  // the nibble formats stream too little per x there to gain on 5 to 8 tiles
+  if (dtype == SWAMP_Q4_0 || dtype == SWAMP_Q4_K)
+    return nx <= 32768 && nt <= (n_cols > 2048 ? 4 : 8);
+  return nx <= (nt >= 3 && n_cols <= 4096 ? 65536 : 32768) && nt <= 8;
 }
 
 // launch_geo with the ragged form when a row's items are not a multiple of
@@ -896,6 +1073,7 @@ size_t kgroup_bytes(uint32_t dtype, int n_tok, int n_rows, int n_cols, int accum
     const int nt = std::min(pl, n_tok - t0);
     if (nt == 1 && !accumulate) continue;  // the decode GEMV
     if (!accumulate && swamp_gemv_tokens_ok(dtype, nt, n_cols)) continue;  // 2 tokens
+    if (xs_route(dtype, nt, n_rows, n_cols)) continue;
     const int nkg = pass_kgroups(nt, n_rows, n_cols);
     if (nkg > 1) ws = std::max(ws, size_t(nkg) * nt * n_rows * sizeof(float));
   }
@@ -977,6 +1155,15 @@ int swamp_launch_gemv_batched(uint32_t dtype, const void *d_w, const float *d_x,
     // item dequantized once (fp16 x, as the passes below)
     if (!accumulate && swamp_gemv_tokens_ok(dtype, a.n_tok, n_cols)) {
       rc = swamp_launch_gemv_tokens(dtype, d_w, a.x, a.y, a.n_tok, n_rows, n_cols, s);
+      continue;
+    }
+    if (xs_route(dtype, a.n_tok, n_rows, n_cols)) {
+      switch (dtype) {
+      case SWAMP_Q4_0: rc = launch_xs<SWAMP_Q4_0>(a, s); break;
+      case SWAMP_Q8_0: rc = launch_xs<SWAMP_Q8_0>(a, s); break;
+      case SWAMP_Q6_K: rc = launch_xs<SWAMP_Q6_K>(a, s); break;
+      default: rc = launch_xs<SWAMP_Q4_K>(a, s); break;
+      }
       continue;
     }
     switch (dtype) {
