@@ -164,16 +164,17 @@ int swamp_launch_split_reduce(const float *d_part, float *d_y, int pieces, size_
 size_t swamp_gemm_scratch_bytes(uint32_t dtype, uint32_t x_type, int m, int n_rows, int n_cols,
                                 size_t limit) {
   if (m <= 0 || n_rows <= 0 || n_cols <= 0) return 0;
-  if (x_type == SWAMP_Q8_0) return swamp_gemm_i8_scratch_bytes(dtype, m, n_rows, n_cols);
+  if (x_type == SWAMP_Q8_0)
+    return swamp::scratch_round(swamp_gemm_i8_scratch_bytes(dtype, m, n_rows, n_cols));
   if (x_type != SWAMP_BF16 || n_cols % kBK != 0) return 0;
   if (swamp_gemm_dq_route(dtype, m, n_rows, n_cols)) {
     const size_t dq = swamp_gemm_dq_scratch_bytes(m, n_rows, n_cols);
     if (dq <= limit || dtype == SWAMP_Q6_K) return dq;
   }
   switch (dtype) {
-    case SWAMP_Q4_0: return plan_bf16<SWAMP_Q4_0>(m, n_rows, n_cols).part_bytes;
-    case SWAMP_Q8_0: return plan_bf16<SWAMP_Q8_0>(m, n_rows, n_cols).part_bytes;
-    case SWAMP_Q4_K: return plan_bf16<SWAMP_Q4_K>(m, n_rows, n_cols).part_bytes;
+    case SWAMP_Q4_0: return swamp::scratch_round(plan_bf16<SWAMP_Q4_0>(m, n_rows, n_cols).part_bytes);
+    case SWAMP_Q8_0: return swamp::scratch_round(plan_bf16<SWAMP_Q8_0>(m, n_rows, n_cols).part_bytes);
+    case SWAMP_Q4_K: return swamp::scratch_round(plan_bf16<SWAMP_Q4_K>(m, n_rows, n_cols).part_bytes);
     case SWAMP_Q6_K: return swamp_gemm_q6k_scratch_bytes(m, n_rows, n_cols);
     default: return 0;
   }

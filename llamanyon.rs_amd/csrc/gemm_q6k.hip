@@ -4,7 +4,7 @@
 #include "gemm_core.hpp"
 
 size_t swamp_gemm_q6k_scratch_bytes(int m, int n_rows, int n_cols) {
-  return plan_bf16<SWAMP_Q6_K>(m, n_rows, n_cols).part_bytes;
+  return swamp::scratch_round(plan_bf16<SWAMP_Q6_K>(m, n_rows, n_cols).part_bytes);
 }
 
 int swamp_launch_gemm_q6k(const void *d_w, const void *d_x, float *d_y, int m, int n_rows,

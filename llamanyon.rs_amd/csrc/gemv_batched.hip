@@ -1077,7 +1077,7 @@ size_t kgroup_bytes(uint32_t dtype, int n_tok, int n_rows, int n_cols, int accum
     const int nkg = pass_kgroups(nt, n_rows, n_cols);
     if (nkg > 1) ws = std::max(ws, size_t(nkg) * nt * n_rows * sizeof(float));
   }
-  return ws;
+  return swamp::scratch_round(ws);
 }
 
 }  // namespace

@@ -103,11 +103,16 @@ const DeviceInfo &device_info();  // current device (initialises it)
 // stream) buffer of stream_workspace or a fixed region the caller names.
 // get() returns nullptr once the region is exhausted; every caller then
 // takes its path without scratch.
+// Bytes a piece takes: the size functions below return whole multiples, so that
+// a region of exactly their size holds what they counted (a region of the bare
+// bytes refused a piece that was no multiple, and its call took the path
+// without scratch).
+constexpr size_t scratch_round(size_t bytes) { return (bytes + 255) & ~size_t(255); }
 struct Scratch {
   uint8_t *base = nullptr;
   size_t cap = 0, used = 0;
   void *get(size_t bytes) {
-    const size_t n = (bytes + 255) & ~size_t(255);
+    const size_t n = scratch_round(bytes);
     if (!base || n > cap - used) return nullptr;
     void *p = base + used;
     used += n;
