@@ -45,10 +45,10 @@
 //    the MFMA work per weight stream), split along K while they fill at
 //    most half the CUs.  Otherwise complete rounds of full tiles; a last round at most
 //    half full runs as twice as many 128-token half tiles (no partial
-//    sums).  Problems of at most half a round split full tiles along K
-//    into up to 8 pieces whose partial tiles go to the stream's workspace
-//    and are summed in piece order by a second kernel (short K: half
-//    tiles; without a workspace: pieces added into zeroed y with float
+//    sums).  Problems of at most half a round split tiles, halves or
+//    quarters of them along K into up to 8 pieces whose partial tiles go to
+//    the stream's workspace and are summed in piece order by a second kernel
+//    (without a workspace: halves, pieces added into zeroed y with float
 //    atomics).
 #pragma once
 
@@ -56,6 +56,7 @@
 #include "swamp_items.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 namespace {
@@ -449,18 +450,21 @@ __device__ __forceinline__ void kstep(f32x16_t (&acc)[kTok], bf16x8_t (&a)[kTok]
 }
 
 // Tile t of the grouped order -> (token tile, weight tile).
-__host__ __device__ inline void tile_coords(int t, int tiles_m, int tiles_n, int &mt, int &nt) {
-  const int grp = t / (kGroup * tiles_n), first = grp * kGroup;
-  const int gs = min(tiles_m - first, kGroup), r = t % (kGroup * tiles_n);
+__host__ __device__ inline void tile_coords(int t, int tiles_m, int tiles_n, int group, int &mt,
+                                            int &nt) {
+  const int grp = t / (group * tiles_n), first = grp * group;
+  const int gs = min(tiles_m - first, group), r = t % (group * tiles_n);
   mt = first + r % gs;
   nt = r / gs;
 }
 
-// Work of one launch: tiles [first, first + count) of the grouped order,
+// Work of one launch: tiles [first, first + count) of the grouped order (tiles
+// of `rows` tokens, `group` token tiles per order group),
 // each as `parts` token parts (1: full tile, 2: halves) x `splits` K pieces.
 struct Work {
   int tiles_m, tiles_n, first, parts, splits, kt_per_split;
   float *part;  // splits > 1: partial sums [piece][M][N] (else added into y atomically)
+  int rows = kBM, group = kGroup;
 };
 
 template <int DT, int kTok>
@@ -485,8 +489,8 @@ __global__ void __launch_bounds__(kThreads, 1)
   const int t = wk.first + u / per_tile, part = (u % per_tile) / wk.splits;
   const int piece = u % wk.splits;
   int mt, nt;
-  tile_coords(t, wk.tiles_m, wk.tiles_n, mt, nt);
-  const int m0 = mt * kBM + part * C::kRows, n0 = nt * kBN;
+  tile_coords(t, wk.tiles_m, wk.tiles_n, wk.group, mt, nt);
+  const int m0 = mt * wk.rows + part * C::kRows, n0 = nt * kBN;
   if (m0 >= M) return;  // second half of a short last token tile (uniform)
   const int KT = K / kBK;
   const int kt0 = piece * wk.kt_per_split, kt1 = min(KT, kt0 + wk.kt_per_split);
@@ -595,7 +599,7 @@ __global__ void zero_tiles_kernel(float *__restrict__ y, int M, int N, int tiles
                                   int first) {
   const int t = first + int(blockIdx.x) / 64;
   int mt, nt;
-  tile_coords(t, tiles_m, tiles_n, mt, nt);
+  tile_coords(t, tiles_m, tiles_n, kGroup, mt, nt);
   const int m = mt * kBM + 4 * (int(blockIdx.x) % 64) + int(threadIdx.x) / 64;
   const int n = nt * kBN + 4 * (int(threadIdx.x) % 64);
   if (m >= M) return;
@@ -622,28 +626,46 @@ int launch_tiles(const uint8_t *w, const uint16_t *x, float *y, int m, int n_row
   return hipGetLastError() == hipSuccess ? SWAMP_OK : SWAMP_ELAUNCH;
 }
 
-// Work decomposition of one bf16 GEMM call (the choice follows measured
-// step times of one tile on one CU -- full 2.0 us, half 1.3 us at 8B
-// shapes -- and 6 TB/s for the partial sums: written, read, y written).
+// Work decomposition of one bf16 GEMM call.
 //  kSmall  at most 64 tokens: 64-token tiles (a quarter of the MFMA work of
 //          a full tile for the same weight stream), split along K into up
 //          to 8 pieces while they fill at most half the CUs;
-//  kSplit  at most half a round of tiles: full tiles split along K into up
-//          to 8 pieces, or 128-token halves (split into up to 4 pieces when
-//          they fill at most half the CUs);
+//  kSplit  at most half a round of tiles: full tiles, 128-token halves or
+//          64-token quarters, those that hold tokens split along K into up to 8
+//          pieces while they fit one round, whichever is estimated fastest;
 //  kRounds full tiles in complete rounds, a last round at most half full as
 //          128-token halves (no partial sums).
 // Split pieces write partial tiles to scratch, summed in piece order by a
 // second kernel (deterministic).  Without scratch the pieces add into
 // zeroed y with float atomics (and kSplit takes halves).
+// The kSplit estimate: measured time of a K step of one tile while a round is
+// full (below; 0.7 of it when few are in flight), 6 us to fill a whole tile's
+// stages and store it, and the partial sums at 6 TB/s, written (partly behind other tiles), read, y written.  It replaced a
+// choice of full tiles or halves in at most 4 pieces, both halves of a tile
+// counted: 100 tokens x 6144 x 4096 Q4_K 31.3 -> 25.4 us (halves, 8 pieces),
+// 150 x 4096 x 14336 57.0 -> 45.1, 70 x 4096 x 4096 27.0 -> 20.3, 256 x 4096 x
+// 4096 29.8 -> 26.1 (quarters), 300 x 6144 x 4096 47.0 -> 35.7 (halves), 120 x
+// 3000 x 28672 88.1 -> 54.5.
 struct GemmPlan {
   enum Kind { kSmall, kSplit, kRounds } kind;
-  bool full;      // kSplit: full tiles (else halves)
+  int parts;      // kSplit: tiles run whole (1), as halves (2) or quarters (4)
   int pieces;     // K pieces (1: none)
   int kps;        // K steps per piece
   int half_pieces, half_kps;  // kSplit fallback without scratch: halves
   size_t part_bytes;          // scratch for the pieces' partial sums
 };
+
+// us of one K step of a whole tile, a half, a quarter, in a full round.
+template <int DT>
+constexpr double step_us(int parts) {
+  return DT == SWAMP_Q6_K   ? (parts == 1 ? 2.65 : 1.68)
+         : DT == SWAMP_Q8_0 ? (parts == 1 ? 2.25 : parts == 2 ? 1.40 : 1.11)
+                            : (parts == 1 ? 2.04 : parts == 2 ? 1.17 : 0.82);
+}
+
+// Scratch of the allocation-free entry point: a split may not grow past it
+// where fewer pieces fit.
+constexpr size_t kFixedScratch = size_t(32) << 20;
 
 template <int DT>
 GemmPlan plan_bf16(int m, int n_rows, int n_cols) {
@@ -656,7 +678,7 @@ GemmPlan plan_bf16(int m, int n_rows, int n_cols) {
     if (DT == SWAMP_Q4_K || DT == SWAMP_Q6_K) kps = (kps + 3) / 4 * 4;
     return kps;
   };
-  GemmPlan p{GemmPlan::kRounds, true, 1, KT, 1, KT, 0};
+  GemmPlan p{GemmPlan::kRounds, 1, 1, KT, 1, KT, 0};
   if (m <= kBM / 4) {
     p.kind = GemmPlan::kSmall;
     int pieces = 2 * tiles <= cus ? std::max(1, std::min({cus / tiles, 8, KT / 8})) : 1;
@@ -664,22 +686,31 @@ GemmPlan plan_bf16(int m, int n_rows, int n_cols) {
     p.pieces = (KT + p.kps - 1) / p.kps;
   } else if (2 * tiles <= cus) {
     p.kind = GemmPlan::kSplit;
-    auto est_us = [&](double step_us, int pieces) {
-      double t_us = double(piece_len(pieces)) * step_us;
-      if (pieces > 1) t_us += (2.0 * pieces + 1.0) * double(mn) * 4.0 / 6e6;
-      return t_us;
-    };
-    const int fs = std::min({cus / tiles, 8, KT / 8});
     const int hs = 4 * tiles <= cus ? std::max(1, std::min({cus / (2 * tiles), 4, KT / 8})) : 1;
     p.half_kps = piece_len(hs);
     p.half_pieces = (KT + p.half_kps - 1) / p.half_kps;
-    p.full = fs >= 2 && est_us(2.0, fs) < est_us(1.3, hs);
-    if (p.full) {
-      p.kps = piece_len(fs);
-      p.pieces = (KT + p.kps - 1) / p.kps;
-    } else {
-      p.kps = p.half_kps;
-      p.pieces = p.half_pieces;
+    const size_t xb = size_t(m) * size_t(n_cols) * 2;  // what a batch of fp32 x adds
+    double best = 0;
+    for (int parts = 1; parts <= (DT == SWAMP_Q6_K ? 2 : 4); parts *= 2) {
+      const int rows = kBM / parts, units = (m + rows - 1) / rows * tiles_n;
+      int last = 0;  // pieces of the previous candidate (rounding repeats them)
+      for (int want = 1; want <= std::max(1, std::min(8, KT / 8)); want++) {
+        const int kps = piece_len(want), pieces = (KT + kps - 1) / kps;
+        if (pieces == last) continue;
+        last = pieces;
+        if (pieces > 1 && units * pieces > cus) break;
+        const size_t part = pieces > 1 ? size_t(pieces) * mn * sizeof(float) : 0;
+        if (pieces > 4 && part + xb + 512 > kFixedScratch && parts > 1) break;
+        const double fill = double(units) * pieces / cus, rounds = std::ceil(fill);
+        double t = 6.0 / parts + kps * step_us<DT>(parts) * rounds * (0.7 + 0.3 * fill / rounds);
+        if (pieces > 1) t += 2.0 + (1.3 * pieces + 1.0) * double(mn) * 4.0 / 6e6;
+        if (best == 0 || t < best) {
+          best = t;
+          p.parts = parts;
+          p.pieces = pieces;
+          p.kps = kps;
+        }
+      }
     }
   }
   p.part_bytes = p.pieces > 1 ? size_t(p.pieces) * mn * sizeof(float) : 0;
@@ -706,22 +737,26 @@ int launch_bf16(const uint8_t *w, const uint16_t *x, float *y, int m, int n_rows
     }
   }
   if (p.kind == GemmPlan::kSplit) {
-    if (p.full && part) {
-      const Work wk{tiles_m, tiles_n, 0, 1, p.pieces, p.kps, part};
-      if (int rc = launch_tiles<DT, 8>(w, x, y, m, n_rows, n_cols, wk, tiles, s)) return rc;
+    if (p.pieces == 1 || part) {
+      // parts are tiles of their own here: a launch of whole tiles' parts, those
+      // past the last token leaving at once, filled some shader engines with
+      // more of the others than they have CUs (300 tokens x 6144 x 4096 Q8_0,
+      // halves in 3 pieces: 216 units of 288 launched took a second round)
+      const int rows = kBM / p.parts, tm = (m + rows - 1) / rows, count = tm * tiles_n;
+      const Work wk{tm, tiles_n, 0, 1, p.pieces, p.kps, part, rows, kGroup * p.parts};
+      int rc = SWAMP_EINVAL;
+      if (p.parts == 1) rc = launch_tiles<DT, 8>(w, x, y, m, n_rows, n_cols, wk, count, s);
+      else if (p.parts == 2) rc = launch_tiles<DT, 4>(w, x, y, m, n_rows, n_cols, wk, count, s);
+      else if constexpr (DT != SWAMP_Q6_K)
+        rc = launch_tiles<DT, 2>(w, x, y, m, n_rows, n_cols, wk, count, s);
+      if (rc || p.pieces == 1) return rc;
       return swamp_launch_split_reduce(part, y, p.pieces, mn, s);
     }
-    // halves: their pieces go to scratch when it is there, else add into
-    // zeroed y
-    const bool use_part = !p.full && part;
-    const int pieces = p.full ? p.half_pieces : p.pieces;
-    const int kps = p.full ? p.half_kps : p.kps;
-    if (pieces > 1 && !use_part)
+    // no scratch: halves, whose pieces add into zeroed y
+    if (p.half_pieces > 1)
       zero_tiles_kernel<<<unsigned(tiles * 64), 256, 0, s>>>(y, m, n_rows, tiles_m, tiles_n, 0);
-    const Work wk{tiles_m, tiles_n, 0, 2, pieces, kps, use_part ? part : nullptr};
-    if (int rc = launch_tiles<DT, 4>(w, x, y, m, n_rows, n_cols, wk, tiles, s)) return rc;
-    if (pieces > 1 && use_part) return swamp_launch_split_reduce(part, y, pieces, mn, s);
-    return SWAMP_OK;
+    const Work wk{tiles_m, tiles_n, 0, 2, p.half_pieces, p.half_kps, nullptr};
+    return launch_tiles<DT, 4>(w, x, y, m, n_rows, n_cols, wk, tiles, s);
   }
   // Full tiles in complete rounds; a last round at most half full as
   // 128-token halves (twice the workgroups, no partial sums).
