@@ -1110,7 +1110,7 @@ int launch_rows(const MatSet &ms, const float *x, const Pro &pro, int n_cols, hi
     // none): 8B Q4_0 qkv 5.97 / 6.31, o_proj 4.55 / 5.08, gate_up 13.79 /
     // 15.14, lm_head 52.2 / 56.5; 70B Q4_K qkv 12.4 / 13.3, gate_up 52.1 /
     // 58.2.  Two sets of four waves (K = 14336) measured slower (down 10.1
-    // / 9.9): their barrier per tile ties the two sets together.
+    // / 9.9): their barrier per tile ties the two sets together,
     if (ipr <= 64) {
       if (ms.sets) return launch_items<DT, 1, kRows, 1, kPro, kX32, 4>(ms, x, pro, n_cols, s);
       return launch_items<DT, 1, kRows, 1, kPro, kX32>(ms, x, pro, n_cols, s);
@@ -1118,6 +1118,16 @@ int launch_rows(const MatSet &ms, const float *x, const Pro &pro, int n_cols, hi
     if (ipr <= 128) {
       if (ms.sets && ms.wpc >= 8) return launch_items<DT, 1, kRows, 2, kPro, kX32, 2>(ms, x, pro, n_cols, s);
       return launch_items<DT, 1, kRows, 2, kPro, kX32>(ms, x, pro, n_cols, s);
+    }
+    // ... except behind the SwiGLU prologue: one set per workgroup reads gate
+    // and up and makes their product twice per CU (115 KB and 14336
+    // exponentials for an 8B down projection).  us, two sets / one: 4096 x
+    // 14336 Q6_K 15.8 / 17.0, Q4_K 10.7 / 12.0, Q4_0 9.8 / 11.2, Q8_0 14.1 /
+    // 16.5; 8192 x 14336 Q4_K 17.1 / 18.0; 2560 x 9216 Q4_K 8.7 / 9.0, but Q6_K
+    // 11.8 / 11.7: too few rows for its single-row tiles.
+    if constexpr (kPro == kProSwiGLU || kPro == kProSwiGLUAcc) {
+      if (ipr <= 256 && ms.sets && ms.wpc >= 8 && (DT != SWAMP_Q6_K || ms.rows[0] >= 3072))
+        return launch_items<DT, 1, kRows, 4, kPro, kX32, 2>(ms, x, pro, n_cols, s);
     }
     if (ipr <= 256) return launch_items<DT, 1, kRows, 4, kPro, kX32>(ms, x, pro, n_cols, s);
     if (ipr <= 512) return launch_items<DT, 1, kRows, 8, kPro, kX32>(ms, x, pro, n_cols, s);
