@@ -663,8 +663,7 @@ constexpr double step_us(int parts) {
                             : (parts == 1 ? 2.04 : parts == 2 ? 1.17 : 0.82);
 }
 
-// Scratch of the allocation-free entry point: a split may not grow past it
-// where fewer pieces fit.
+// Scratch of the allocation-free small-batch entry point.
 constexpr size_t kFixedScratch = size_t(32) << 20;
 
 template <int DT>
@@ -689,7 +688,17 @@ GemmPlan plan_bf16(int m, int n_rows, int n_cols) {
     const int hs = 4 * tiles <= cus ? std::max(1, std::min({cus / (2 * tiles), 4, KT / 8})) : 1;
     p.half_kps = piece_len(hs);
     p.half_pieces = (KT + p.half_kps - 1) / p.half_kps;
-    const size_t xb = size_t(m) * size_t(n_cols) * 2;  // what a batch of fp32 x adds
+    // Calls that the allocation-free entry point's scratch holds keep fitting: a
+    // split takes no more than that leaves beside the bf16 x, or than the
+    // simpler choice of whole tiles or halves (2.0 and 1.3 us a step) would.
+    const int fs = std::min({cus / tiles, 8, KT / 8});
+    auto plain_us = [&](double step, int n) {
+      return piece_len(n) * step + (n > 1 ? (2.0 * n + 1.0) * double(mn) * 4.0 / 6e6 : 0.0);
+    };
+    const int plain = piece_len(fs >= 2 && plain_us(2.0, fs) < plain_us(1.3, hs) ? fs : hs);
+    const size_t xb = size_t(m) * size_t(n_cols) * 2 + 512;
+    const size_t cap = std::max(plain < KT ? size_t((KT + plain - 1) / plain) * mn * sizeof(float) : 0,
+                                kFixedScratch - std::min(xb, kFixedScratch));
     double best = 0;
     for (int parts = 1; parts <= (DT == SWAMP_Q6_K ? 2 : 4); parts *= 2) {
       const int rows = kBM / parts, units = (m + rows - 1) / rows * tiles_n;
@@ -700,7 +709,7 @@ GemmPlan plan_bf16(int m, int n_rows, int n_cols) {
         last = pieces;
         if (pieces > 1 && units * pieces > cus) break;
         const size_t part = pieces > 1 ? size_t(pieces) * mn * sizeof(float) : 0;
-        if (pieces > 4 && part + xb + 512 > kFixedScratch && parts > 1) break;
+        if (part > cap) break;
         const double fill = double(units) * pieces / cus, rounds = std::ceil(fill);
         double t = 6.0 / parts + kps * step_us<DT>(parts) * rounds * (0.7 + 0.3 * fill / rounds);
         if (pieces > 1) t += 2.0 + (1.3 * pieces + 1.0) * double(mn) * 4.0 / 6e6;
