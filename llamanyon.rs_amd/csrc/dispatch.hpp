@@ -1,0 +1,176 @@
+// dispatch.hpp -- the rules on sizes that choose between the library's
+// kernels and work decompositions: host arithmetic on the shape and the number
+// of CUs alone, no HIP, so that they compile and can be checked without a GPU.
+#pragma once
+
+#include <stddef.h>
+#include <stdint.h>
+
+#include <algorithm>
+#include <cmath>
+
+#include "swamp_qmm.h"
+
+namespace swamp {
+
+// Full tile (tokens, weight rows) and K step of the fused bf16 GEMM.
+constexpr int kGemmTokens = 256, kGemmRows = 256, kGemmK = 64;
+
+// Work decomposition of one bf16 GEMM call.
+//  kSmall  at most 64 tokens: 64-token tiles (a quarter of the MFMA work of
+//          a full tile for the same weight stream), split along K into up
+//          to 8 pieces while they fill at most half the CUs;
+//  kSplit  at most half a round of tiles: full tiles, 128-token halves or
+//          64-token quarters, those that hold tokens split along K into up to 8
+//          pieces while they fit one round, whichever is estimated fastest;
+//  kRounds full tiles in complete rounds, a last round at most half full as
+//          128-token halves (no partial sums).
+// Split pieces write partial tiles to scratch, summed in piece order by a
+// second kernel (deterministic).  Without scratch the pieces add into
+// zeroed y with float atomics (and kSplit takes halves).
+// The kSplit estimate: measured time of a K step of one tile while a round is
+// full (below; 0.7 of it when few are in flight), 6 us to fill a whole tile's
+// stages and store it, and the partial sums at 6 TB/s, written (partly behind other tiles), read, y written.  It replaced a
+// choice of full tiles or halves in at most 4 pieces, both halves of a tile
+// counted: 100 tokens x 6144 x 4096 Q4_K 31.3 -> 25.4 us (halves, 8 pieces),
+// 150 x 4096 x 14336 57.0 -> 45.1, 70 x 4096 x 4096 27.0 -> 20.3, 256 x 4096 x
+// 4096 29.8 -> 26.1 (quarters), 300 x 6144 x 4096 47.0 -> 35.7 (halves), 120 x
+// 3000 x 28672 88.1 -> 54.5.
+struct GemmPlan {
+  enum Kind { kSmall, kSplit, kRounds } kind;
+  int parts;      // kSplit: tiles run whole (1), as halves (2) or quarters (4)
+  int pieces;     // K pieces (1: none)
+  int kps;        // K steps per piece
+  int half_pieces, half_kps;  // kSplit fallback without scratch: halves
+  size_t part_bytes;          // scratch for the pieces' partial sums
+};
+
+// us of one K step of a whole tile, a half, a quarter, in a full round.
+constexpr double gemm_step_us(uint32_t dt, int parts) {
+  return dt == SWAMP_Q6_K   ? (parts == 1 ? 2.65 : 1.68)
+         : dt == SWAMP_Q8_0 ? (parts == 1 ? 2.25 : parts == 2 ? 1.40 : 1.11)
+                            : (parts == 1 ? 2.04 : parts == 2 ? 1.17 : 0.82);
+}
+
+inline GemmPlan plan_gemm_bf16(uint32_t dt, int m, int n_rows, int n_cols, int cus) {
+  constexpr int kBM = kGemmTokens;
+  const int tiles_m = (m + kBM - 1) / kBM, tiles_n = (n_rows + kGemmRows - 1) / kGemmRows;
+  const int tiles = tiles_m * tiles_n, KT = n_cols / kGemmK;
+  const size_t mn = size_t(m) * size_t(n_rows);
+  auto piece_len = [&](int splits) {  // K steps per piece (whole 256-weight blocks)
+    int kps = (KT + splits - 1) / splits;
+    if (dt == SWAMP_Q4_K || dt == SWAMP_Q6_K) kps = (kps + 3) / 4 * 4;
+    return kps;
+  };
+  GemmPlan p{GemmPlan::kRounds, 1, 1, KT, 1, KT, 0};
+  if (m <= kBM / 4) {
+    p.kind = GemmPlan::kSmall;
+    int pieces = 2 * tiles <= cus ? std::max(1, std::min({cus / tiles, 8, KT / 8})) : 1;
+    p.kps = piece_len(pieces);
+    p.pieces = (KT + p.kps - 1) / p.kps;
+  } else if (2 * tiles <= cus) {
+    p.kind = GemmPlan::kSplit;
+    const int hs = 4 * tiles <= cus ? std::max(1, std::min({cus / (2 * tiles), 4, KT / 8})) : 1;
+    p.half_kps = piece_len(hs);
+    p.half_pieces = (KT + p.half_kps - 1) / p.half_kps;
+    // Calls that the allocation-free entry point's scratch holds keep fitting: a
+    // split takes no more than that leaves beside the bf16 x, or than the
+    // simpler choice of whole tiles or halves (2.0 and 1.3 us a step) would.
+    const int fs = std::min({cus / tiles, 8, KT / 8});
+    auto plain_us = [&](double step, int n) {
+      return piece_len(n) * step + (n > 1 ? (2.0 * n + 1.0) * double(mn) * 4.0 / 6e6 : 0.0);
+    };
+    const int plain = piece_len(fs >= 2 && plain_us(2.0, fs) < plain_us(1.3, hs) ? fs : hs);
+    const size_t xb = size_t(m) * size_t(n_cols) * 2 + 512;
+    const size_t cap = std::max(plain < KT ? size_t((KT + plain - 1) / plain) * mn * sizeof(float) : 0,
+                                SWAMP_NOALLOC_SCRATCH_BYTES -
+                                    std::min(xb, SWAMP_NOALLOC_SCRATCH_BYTES));
+    double best = 0;
+    for (int parts = 1; parts <= (dt == SWAMP_Q6_K ? 2 : 4); parts *= 2) {
+      const int rows = kBM / parts, units = (m + rows - 1) / rows * tiles_n;
+      int last = 0;  // pieces of the previous candidate (rounding repeats them)
+      for (int want = 1; want <= std::max(1, std::min(8, KT / 8)); want++) {
+        const int kps = piece_len(want), pieces = (KT + kps - 1) / kps;
+        if (pieces == last) continue;
+        last = pieces;
+        if (pieces > 1 && units * pieces > cus) break;
+        const size_t part = pieces > 1 ? size_t(pieces) * mn * sizeof(float) : 0;
+        if (part > cap) break;
+        const double fill = double(units) * pieces / cus, rounds = std::ceil(fill);
+        double t =
+            6.0 / parts + kps * gemm_step_us(dt, parts) * rounds * (0.7 + 0.3 * fill / rounds);
+        if (pieces > 1) t += 2.0 + (1.3 * pieces + 1.0) * double(mn) * 4.0 / 6e6;
+        if (best == 0 || t < best) {
+          best = t;
+          p.parts = parts;
+          p.pieces = pieces;
+          p.kps = kps;
+        }
+      }
+    }
+  }
+  p.part_bytes = p.pieces > 1 ? size_t(p.pieces) * mn * sizeof(float) : 0;
+  return p;
+}
+
+// Shapes the fused Q6_K GEMM takes: it reads rows of whole block pairs
+// (dword-aligned); at most 64 tokens it would run its 64-token tiles, where the
+// dequantization of a tile's weights is not spread over enough tokens.
+inline bool q6k_gemm_fusable(int m, int n_cols) { return m > 64 && n_cols % 512 == 0; }
+
+// Whether a bf16 GEMM dequantizes its weights to memory once and multiplies
+// them with the plain bf16 GEMM, instead of the fused kernel.
+inline bool gemm_dequantize_once(uint32_t dtype, int m, int n_rows, int n_cols, int cus) {
+  const long tiles = long((m + 255) / 256) * long((n_rows + 255) / 256);
+  if (dtype == SWAMP_Q6_K) {
+    // Q6_K's fused dequantization takes twice the vector work of the others
+    // per matrix instruction; this route instead writes and re-reads 2 bytes
+    // per weight.  Fused where that traffic counts most: few tokens, or long
+    // rows whose tiles split along K -- but not where too few tiles are left
+    // to split.  us, fused / this route: 512 x 28672 x 4096 158 / 182, 600
+    // 247 / 247, 1000 298 / 289; 512 x 6144 x 4096 66 / 66, 1000 103 / 88;
+    // 777 x 4096 x 14336 150 / 187, 1500 254 / 295, 2048 286 / 312; 200 x
+    // 3000 x 5120 (12 tiles) 40 / 32, 70 x 2048 x 14336 (8 tiles) 57 / 46.
+    if (!q6k_gemm_fusable(m, n_cols)) return true;
+    const bool fused = 16 * tiles >= cus && (m <= 512 || (2 * tiles <= cus && n_cols >= 8192));
+    return !fused;
+  }
+  // The fused kernel reads 0.56-1.06 bytes per weight per tile, the plain
+  // bf16 GEMM 2 (its loads from L2 bound it, not the dequantization), so the
+  // fused kernel is faster wherever its 256 x 256 tiles fill whole rounds of
+  // the CUs or split along K.  Between half a round and one round they leave
+  // CUs idle, and the plain GEMM's 256-token x 192-row tiles fill them: this
+  // route, once every weight meets enough tokens to repay the dequantization.
+  // `bench.py --route-crossover` (8B shapes, us, fused / this route, Q4_0):
+  // 2048 tokens qkv 113.1 / 109.4, gate_up 514.0 / 599.1, down 253.0 / 324.4,
+  // o_proj 76.5 / 84.9; Q8_0 qkv 128.7 / 112.8; Q4_K qkv 116.8 / 111.4.
+  if (m < 1024 || n_cols < 1024) return false;
+  return 2 * tiles > cus && tiles < cus;
+}
+
+// Rows of a 16-row tile of the small-batch kernels.
+constexpr int kBatchTileRows = 16;
+
+// Passes for gemv_xs_kernel: x read once per workgroup, so few tokens times a
+// short row, and tiles for at most one round of workgroups.  us, the kernel
+// above / gemv_xs: Q4_K 4096 x 4096 at 3, 5, 8 tokens 7.2 / 6.4, 9.6 / 7.0,
+// 9.6 / 9.4, at 12 9.7 / 13.4; Q6_K 1024 x 4096 at 5 10.6 / 7.7; Q8_0
+// 4096 x 3072 at 5 8.5 / 6.7; rows of 14336 weights 14.5 / 22.0.  More rows
+// than 4096 take 2 to 8 tiles per workgroup, whose 8 waves are all busy when
+// the row is whole 2048-weight passes: Q4_K 14336 x 4096 at 5 14.8 / 13.2,
+// 9000 x 3072 10.5 / 10.6, 28672 x 4096 at 8 21.1 / 21.6; Q8_0 28672 x 4096 at
+// 5 and 16 32.8 / 31.1, 36.6 / 35.5; 128256 x 4096 at 5 108 / 120.
+inline bool small_batch_in_registers(uint32_t dtype, int n_tok, int n_rows, int n_cols, int cus) {
+  const int n_tiles = (n_rows + kBatchTileRows - 1) / kBatchTileRows;
+  const int nt = (n_tiles + cus - 1) / cus;  // tiles per workgroup
+  const long nx = long(n_tok) * n_cols;
+  if (n_tok > 16 || n_cols % 256 != 0) return false;
+  if (nt <= 1) return n_cols <= 4096 && nx <= 32768;
+  if (n_cols % 2048 != 0) return false;
+  // the nibble formats stream too little per x there to gain on 5 to 8 tiles
+  if (dtype == SWAMP_Q4_0 || dtype == SWAMP_Q4_K)
+    return nx <= 32768 && nt <= (n_cols > 2048 ? 4 : 8);
+  return nx <= (nt >= 3 && n_cols <= 4096 ? 65536 : 32768) && nt <= 8;
+}
+
+}  // namespace swamp

@@ -52,15 +52,16 @@
 //    atomics).
 #pragma once
 
+#include "dispatch.hpp"
 #include "swamp_common.hpp"
 #include "swamp_items.hpp"
 
 #include <algorithm>
-#include <cmath>
 #include <mutex>
 
 namespace {
 
+using swamp::GemmPlan;
 using swamp::q4k_scales;
 using swamp::shr16;
 
@@ -70,7 +71,8 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4v_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x3v_t __attribute__((ext_vector_type(3)));
 
-constexpr int kBM = 256, kBN = 256, kBK = 64;  // full tile and K step
+// full tile and K step
+constexpr int kBM = swamp::kGemmTokens, kBN = swamp::kGemmRows, kBK = swamp::kGemmK;
 constexpr int kThreads = 512, kWaves = 8;
 constexpr int kStages = 5;                     // activation stages
 constexpr int kGroup = 4;                      // token tiles per order group
@@ -626,104 +628,9 @@ int launch_tiles(const uint8_t *w, const uint16_t *x, float *y, int m, int n_row
   return hipGetLastError() == hipSuccess ? SWAMP_OK : SWAMP_ELAUNCH;
 }
 
-// Work decomposition of one bf16 GEMM call.
-//  kSmall  at most 64 tokens: 64-token tiles (a quarter of the MFMA work of
-//          a full tile for the same weight stream), split along K into up
-//          to 8 pieces while they fill at most half the CUs;
-//  kSplit  at most half a round of tiles: full tiles, 128-token halves or
-//          64-token quarters, those that hold tokens split along K into up to 8
-//          pieces while they fit one round, whichever is estimated fastest;
-//  kRounds full tiles in complete rounds, a last round at most half full as
-//          128-token halves (no partial sums).
-// Split pieces write partial tiles to scratch, summed in piece order by a
-// second kernel (deterministic).  Without scratch the pieces add into
-// zeroed y with float atomics (and kSplit takes halves).
-// The kSplit estimate: measured time of a K step of one tile while a round is
-// full (below; 0.7 of it when few are in flight), 6 us to fill a whole tile's
-// stages and store it, and the partial sums at 6 TB/s, written (partly behind other tiles), read, y written.  It replaced a
-// choice of full tiles or halves in at most 4 pieces, both halves of a tile
-// counted: 100 tokens x 6144 x 4096 Q4_K 31.3 -> 25.4 us (halves, 8 pieces),
-// 150 x 4096 x 14336 57.0 -> 45.1, 70 x 4096 x 4096 27.0 -> 20.3, 256 x 4096 x
-// 4096 29.8 -> 26.1 (quarters), 300 x 6144 x 4096 47.0 -> 35.7 (halves), 120 x
-// 3000 x 28672 88.1 -> 54.5.
-struct GemmPlan {
-  enum Kind { kSmall, kSplit, kRounds } kind;
-  int parts;      // kSplit: tiles run whole (1), as halves (2) or quarters (4)
-  int pieces;     // K pieces (1: none)
-  int kps;        // K steps per piece
-  int half_pieces, half_kps;  // kSplit fallback without scratch: halves
-  size_t part_bytes;          // scratch for the pieces' partial sums
-};
-
-// us of one K step of a whole tile, a half, a quarter, in a full round.
-template <int DT>
-constexpr double step_us(int parts) {
-  return DT == SWAMP_Q6_K   ? (parts == 1 ? 2.65 : 1.68)
-         : DT == SWAMP_Q8_0 ? (parts == 1 ? 2.25 : parts == 2 ? 1.40 : 1.11)
-                            : (parts == 1 ? 2.04 : parts == 2 ? 1.17 : 0.82);
-}
-
-// Scratch of the allocation-free small-batch entry point.
-constexpr size_t kFixedScratch = size_t(32) << 20;
-
 template <int DT>
 GemmPlan plan_bf16(int m, int n_rows, int n_cols) {
-  const int tiles_m = (m + kBM - 1) / kBM, tiles_n = (n_rows + kBN - 1) / kBN;
-  const int tiles = tiles_m * tiles_n, KT = n_cols / kBK;
-  const int cus = swamp::device_info().num_cus;
-  const size_t mn = size_t(m) * size_t(n_rows);
-  auto piece_len = [&](int splits) {  // K steps per piece (whole 256-weight blocks)
-    int kps = (KT + splits - 1) / splits;
-    if (DT == SWAMP_Q4_K || DT == SWAMP_Q6_K) kps = (kps + 3) / 4 * 4;
-    return kps;
-  };
-  GemmPlan p{GemmPlan::kRounds, 1, 1, KT, 1, KT, 0};
-  if (m <= kBM / 4) {
-    p.kind = GemmPlan::kSmall;
-    int pieces = 2 * tiles <= cus ? std::max(1, std::min({cus / tiles, 8, KT / 8})) : 1;
-    p.kps = piece_len(pieces);
-    p.pieces = (KT + p.kps - 1) / p.kps;
-  } else if (2 * tiles <= cus) {
-    p.kind = GemmPlan::kSplit;
-    const int hs = 4 * tiles <= cus ? std::max(1, std::min({cus / (2 * tiles), 4, KT / 8})) : 1;
-    p.half_kps = piece_len(hs);
-    p.half_pieces = (KT + p.half_kps - 1) / p.half_kps;
-    // Calls that the allocation-free entry point's scratch holds keep fitting: a
-    // split takes no more than that leaves beside the bf16 x, or than the
-    // simpler choice of whole tiles or halves (2.0 and 1.3 us a step) would.
-    const int fs = std::min({cus / tiles, 8, KT / 8});
-    auto plain_us = [&](double step, int n) {
-      return piece_len(n) * step + (n > 1 ? (2.0 * n + 1.0) * double(mn) * 4.0 / 6e6 : 0.0);
-    };
-    const int plain = piece_len(fs >= 2 && plain_us(2.0, fs) < plain_us(1.3, hs) ? fs : hs);
-    const size_t xb = size_t(m) * size_t(n_cols) * 2 + 512;
-    const size_t cap = std::max(plain < KT ? size_t((KT + plain - 1) / plain) * mn * sizeof(float) : 0,
-                                kFixedScratch - std::min(xb, kFixedScratch));
-    double best = 0;
-    for (int parts = 1; parts <= (DT == SWAMP_Q6_K ? 2 : 4); parts *= 2) {
-      const int rows = kBM / parts, units = (m + rows - 1) / rows * tiles_n;
-      int last = 0;  // pieces of the previous candidate (rounding repeats them)
-      for (int want = 1; want <= std::max(1, std::min(8, KT / 8)); want++) {
-        const int kps = piece_len(want), pieces = (KT + kps - 1) / kps;
-        if (pieces == last) continue;
-        last = pieces;
-        if (pieces > 1 && units * pieces > cus) break;
-        const size_t part = pieces > 1 ? size_t(pieces) * mn * sizeof(float) : 0;
-        if (part > cap) break;
-        const double fill = double(units) * pieces / cus, rounds = std::ceil(fill);
-        double t = 6.0 / parts + kps * step_us<DT>(parts) * rounds * (0.7 + 0.3 * fill / rounds);
-        if (pieces > 1) t += 2.0 + (1.3 * pieces + 1.0) * double(mn) * 4.0 / 6e6;
-        if (best == 0 || t < best) {
-          best = t;
-          p.parts = parts;
-          p.pieces = pieces;
-          p.kps = kps;
-        }
-      }
-    }
-  }
-  p.part_bytes = p.pieces > 1 ? size_t(p.pieces) * mn * sizeof(float) : 0;
-  return p;
+  return swamp::plan_gemm_bf16(DT, m, n_rows, n_cols, swamp::device_info().num_cus);
 }
 
 template <int DT>

@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <cstdlib>
 
+#include "dispatch.hpp"
 #include "swamp_common.hpp"
 
 size_t swamp_gemm_bb_scratch_bytes(int m, int n_rows, int n_cols);
@@ -53,38 +54,11 @@ int route_forced() {  // tuning override, read per call: SWAMP_GEMM_ROUTE=fused|
 }  // namespace
 
 bool swamp_gemm_dq_route(uint32_t dtype, int m, int n_rows, int n_cols) {
-  // the fused Q6_K kernel reads rows of whole block pairs (dword-aligned); at
-  // most 64 tokens it would run its 64-token tiles, where the dequantization
-  // of a tile's weights is not spread over enough tokens
-  if (dtype == SWAMP_Q6_K && (m <= 64 || n_cols % 512 != 0)) return true;
+  if (dtype == SWAMP_Q6_K && !swamp::q6k_gemm_fusable(m, n_cols)) return true;
   if (dtype != SWAMP_Q4_0 && dtype != SWAMP_Q8_0 && dtype != SWAMP_Q4_K && dtype != SWAMP_Q6_K)
     return false;
   if (int f = route_forced()) return f == 2;
-  const int cus = swamp::device_info().num_cus;
-  const long tiles = long((m + 255) / 256) * long((n_rows + 255) / 256);
-  if (dtype == SWAMP_Q6_K) {
-    // Q6_K's fused dequantization takes twice the vector work of the others
-    // per matrix instruction; this route instead writes and re-reads 2 bytes
-    // per weight.  Fused where that traffic counts most: few tokens, or long
-    // rows whose tiles split along K -- but not where too few tiles are left
-    // to split.  us, fused / this route: 512 x 28672 x 4096 158 / 182, 600
-    // 247 / 247, 1000 298 / 289; 512 x 6144 x 4096 66 / 66, 1000 103 / 88;
-    // 777 x 4096 x 14336 150 / 187, 1500 254 / 295, 2048 286 / 312; 200 x
-    // 3000 x 5120 (12 tiles) 40 / 32, 70 x 2048 x 14336 (8 tiles) 57 / 46.
-    const bool fused = 16 * tiles >= cus && (m <= 512 || (2 * tiles <= cus && n_cols >= 8192));
-    return !fused;
-  }
-  // The fused kernel reads 0.56-1.06 bytes per weight per tile, the plain
-  // bf16 GEMM 2 (its loads from L2 bound it, not the dequantization), so the
-  // fused kernel is faster wherever its 256 x 256 tiles fill whole rounds of
-  // the CUs or split along K.  Between half a round and one round they leave
-  // CUs idle, and the plain GEMM's 256-token x 192-row tiles fill them: this
-  // route, once every weight meets enough tokens to repay the dequantization.
-  // `bench.py --route-crossover` (8B shapes, us, fused / this route, Q4_0):
-  // 2048 tokens qkv 113.1 / 109.4, gate_up 514.0 / 599.1, down 253.0 / 324.4,
-  // o_proj 76.5 / 84.9; Q8_0 qkv 128.7 / 112.8; Q4_K qkv 116.8 / 111.4.
-  if (m < 1024 || n_cols < 1024) return false;
-  return 2 * tiles > cus && tiles < cus;
+  return swamp::gemm_dequantize_once(dtype, m, n_rows, n_cols, swamp::device_info().num_cus);
 }
 
 size_t swamp_gemm_dq_scratch_bytes(int m, int n_rows, int n_cols) {

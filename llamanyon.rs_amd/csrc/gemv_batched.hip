@@ -34,6 +34,7 @@
 #include <cstdlib>
 #include <mutex>
 
+#include "dispatch.hpp"
 #include "swamp_common.hpp"
 #include "swamp_items.hpp"
 
@@ -49,7 +50,7 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 constexpr int kWaves = 16;      // waves per workgroup, one workgroup per CU
 constexpr int kThreads = kWaves * 64;
 constexpr int kTok = 64;        // tokens per pass: up to 4 groups of 16 (MFMA M)
-constexpr int kRowsTile = 16;   // rows per tile (MFMA N)
+constexpr int kRowsTile = swamp::kBatchTileRows;  // rows per tile (MFMA N)
 constexpr int kJmax = 2;        // tiles per wave whose accumulators stay in registers
 constexpr int kXLdsMax = 139264;             // activation bytes in LDS (one K phase)
 constexpr int kSlotBytes = kWaves * 16 * 16 * 4;  // one 16x16 fp32 partial per wave
@@ -903,27 +904,9 @@ int launch_xs(const Args &a, hipStream_t s) {
   if (nt <= 4) return launch_xs_t<DT, 4>(a, nt, s);
   return launch_xs_t<DT, 8>(a, nt, s);
 }
-// Passes for gemv_xs_kernel: x read once per workgroup, so few tokens times a
-// short row, and tiles for at most one round of workgroups.  us, the kernel
-// above / gemv_xs: Q4_K 4096 x 4096 at 3, 5, 8 tokens 7.2 / 6.4, 9.6 / 7.0,
-// 9.6 / 9.4, at 12 9.7 / 13.4; Q6_K 1024 x 4096 at 5 10.6 / 7.7; Q8_0
-// 4096 x 3072 at 5 8.5 / 6.7; rows of 14336 weights 14.5 / 22.0.  More rows
-// than 4096 take 2 to 8 tiles per workgroup, whose 8 waves are all busy when
-// the row is whole 2048-weight passes: Q4_K 14336 x 4096 at 5 14.8 / 13.2,
-// 9000 x 3072 10.5 / 10.6, 28672 x 4096 at 8 21.1 / 21.6; Q8_0 28672 x 4096 at
-// 5 and 16 32.8 / 31.1, 36.6 / 35.5; 128256 x 4096 at 5 108 / 120.
 bool xs_route(uint32_t dtype, int n_tok, int n_rows, int n_cols) {
-  const int n_tiles = (n_rows + kRowsTile - 1) / kRowsTile;
-  const int cus = swamp::device_info().num_cus;
-  const int nt = (n_tiles + cus - 1) / cus;  // tiles per workgroup
-  const long nx = long(n_tok) * n_cols;
-  if (n_tok > 16 || n_cols % 256 != 0) return false;
-  if (nt <= 1) return n_cols <= 4096 && nx <= 32768;
-  if (n_cols % 2048 != 0) return false;
-  // the nibble formats stream too little per x there to gain on 5 to 8 tiles
-  if (dtype == SWAMP_Q4_0 || dtype == SWAMP_Q4_K)
-    return nx <= 32768 && nt <= (n_cols > 2048 ? 4 : 8);
-  return nx <= (nt >= 3 && n_cols <= 4096 ? 65536 : 32768) && nt <= 8;
+  return swamp::small_batch_in_registers(dtype, n_tok, n_rows, n_cols,
+                                         swamp::device_info().num_cus);
 }
 
 // launch_geo with the ragged form when a row's items are not a multiple of
