@@ -151,26 +151,48 @@ inline bool gemm_dequantize_once(uint32_t dtype, int m, int n_rows, int n_cols, 
 // Rows of a 16-row tile of the small-batch kernels.
 constexpr int kBatchTileRows = 16;
 
-// Passes for gemv_xs_kernel: x read once per workgroup, so few tokens times a
-// short row, and tiles for at most one round of workgroups.  us, the kernel
-// above / gemv_xs: Q4_K 4096 x 4096 at 3, 5, 8 tokens 7.2 / 6.4, 9.6 / 7.0,
-// 9.6 / 9.4, at 12 9.7 / 13.4; Q6_K 1024 x 4096 at 5 10.6 / 7.7; Q8_0
-// 4096 x 3072 at 5 8.5 / 6.7; rows of 14336 weights 14.5 / 22.0.  More rows
-// than 4096 take 2 to 8 tiles per workgroup, whose 8 waves are all busy when
-// the row is whole 2048-weight passes: Q4_K 14336 x 4096 at 5 14.8 / 13.2,
-// 9000 x 3072 10.5 / 10.6, 28672 x 4096 at 8 21.1 / 21.6; Q8_0 28672 x 4096 at
-// 5 and 16 32.8 / 31.1, 36.6 / 35.5; 128256 x 4096 at 5 108 / 120.
+// Small-batch passes that take gemv_xs_kernel, which loads each wave's share of
+// x into registers, instead of gemv_batched_kernel, which stages x through LDS.
+// Every workgroup of the former converts all of x for itself, so it is faster
+// only while tokens times row length are few.  Measured over 10000 shapes, 1 to
+// 16 tokens x 256 to 32768 rows x 256 to 32768 weights; us, staged / registers:
+//  * One tile per workgroup (rows <= 16 x the CUs): 16 waves take up to 4096
+//    weights in one pass (rows of 14336 lose, 14.5 / 22.0).  Q6_K gains up to 32768 x
+//    values: 1024 x 4096 at 5 tokens 10.5 / 8.4, 4096 x 2048 at 16 10.3 / 8.9.
+//    Q8_0 4096 x 2048 at 14 9.6 / 9.0, but 4096 x 2560 at 12 8.7 / 9.1; Q4_0
+//    4096 x 2048 at 12 8.1 / 7.6, but 4096 x 4096 at 8 8.2 / 8.8.
+//  * Q4_K's scale unpacking makes the line fall faster than the token count
+//    rises: 4096 x 4096 at 5 8.0 / 7.5, at 6 8.1 / 8.4, at 8 8.1 / 10.0; 4096 x
+//    2048 at 8 7.8 / 7.7, at 16 8.6 / 11.8.  Rows that are not whole 1024-weight
+//    granules of the staged kernel leave more room: 4096 x 1280 at 12 8.1 / 7.7.
+//  * Rows of 256 weights gain nothing (5.1 / 5.3).
+//  * More rows take 2 to 8 tiles per workgroup, whose 8 waves are all busy when
+//    the row is whole 2048-weight passes; each pass beyond the second costs
+//    more than staging: Q4_K 14336 x 4096 at 5 16.0 / 14.4, but 5120 x 8192 at
+//    4 12.7 / 16.2 and 5120 x 14336 at 2 16.7 / 23.4; Q4_0 5120 x 28672 at 1
+//    25.0 / 39.0.  Q8_0 and Q6_K stream enough weights behind their x for that
+//    at 4 tiles: 14336 x 8192 at 4 34.9 / 33.4, 14336 x 6144 at 5 27.6 / 25.2.
+//  * 5 and 6 tiles run the instance of 8, whose idle tiles cost the nibble
+//    formats more than they gain: 20480 x 2048 at 16 Q4_K 13.4 / 14.8, but 28672
+//    x 2048 at 8 14.9 / 13.8.  So does a single token on 4 tiles: 13.7 / 14.5.
 inline bool small_batch_in_registers(uint32_t dtype, int n_tok, int n_rows, int n_cols, int cus) {
   const int n_tiles = (n_rows + kBatchTileRows - 1) / kBatchTileRows;
   const int nt = (n_tiles + cus - 1) / cus;  // tiles per workgroup
   const long nx = long(n_tok) * n_cols;
-  if (n_tok > 16 || n_cols % 256 != 0) return false;
-  if (nt <= 1) return n_cols <= 4096 && nx <= 32768;
-  if (n_cols % 2048 != 0) return false;
-  // the nibble formats stream too little per x there to gain on 5 to 8 tiles
-  if (dtype == SWAMP_Q4_0 || dtype == SWAMP_Q4_K)
-    return nx <= 32768 && nt <= (n_cols > 2048 ? 4 : 8);
-  return nx <= (nt >= 3 && n_cols <= 4096 ? 65536 : 32768) && nt <= 8;
+  const bool nibbles = dtype == SWAMP_Q4_0 || dtype == SWAMP_Q4_K;
+  if (n_tok > 16 || n_cols % 256 != 0 || n_cols < 512) return false;
+  if (nt <= 1) {
+    if (n_cols > 4096) return false;
+    if (dtype == SWAMP_Q4_K)
+      return nx <= 21504 && nx * n_tok <= (n_cols % 1024 ? 196608 : 131072);
+    return nx <= (dtype == SWAMP_Q6_K ? 32768 : dtype == SWAMP_Q8_0 ? 28672 : 27648);
+  }
+  if (nt > 8 || n_cols % 2048 != 0) return false;
+  if (nibbles)
+    return n_cols <= (nt <= 4 ? 4096 : 2048) && nt != 5 && nt != 6 &&
+           n_tok >= (nt <= 3 ? 2 : 3) && nx <= (nt == 3 || nt == 4 ? 32768 : 28672);
+  if (n_cols <= 4096) return nx <= (nt >= 3 ? 57344 : 32768);
+  return n_cols <= 8192 && nt >= 4 && nt <= (dtype == SWAMP_Q8_0 ? 5 : 4) && nx <= 32768;
 }
 
 }  // namespace swamp

@@ -36,3 +36,39 @@ def test_bench_route_labels_follow_the_rule(rules, bench):
                     assert label.startswith("dequantize-once") == want, (dt, m, rows, cols, label)
                     seen.add((dt == Q6_K, want))
     assert len(seen) == 4
+
+
+# (dtype, tokens, rows, weights per row, us staged, us in registers), measured on
+# an MI355X over rotating weights
+SMALL_BATCH = [
+    (Q4_0, 1, 4096, 256, 5.10, 5.25), (Q4_0, 5, 4096, 4096, 7.97, 7.55),
+    (Q4_0, 8, 4096, 4096, 8.16, 8.81), (Q4_0, 12, 4096, 2048, 8.07, 7.56),
+    (Q4_0, 8, 14336, 2048, 10.86, 9.50), (Q4_0, 5, 14336, 4096, 15.59, 14.06),
+    (Q4_0, 3, 5120, 8192, 12.30, 15.51), (Q4_0, 1, 16384, 4096, 13.85, 14.56),
+    (Q4_0, 12, 28672, 2048, 15.45, 14.41), (Q4_0, 1, 5120, 28672, 24.97, 38.96),
+    (Q8_0, 5, 4096, 4096, 9.92, 8.68), (Q8_0, 14, 4096, 2048, 9.58, 9.00),
+    (Q8_0, 12, 4096, 2560, 8.72, 9.12), (Q8_0, 5, 14336, 4096, 22.42, 19.67),
+    (Q8_0, 14, 14336, 4096, 24.41, 22.79), (Q8_0, 4, 5120, 8192, 17.69, 20.71),
+    (Q8_0, 1, 5120, 28672, 38.38, 55.86), (Q8_0, 3, 5120, 10240, 20.48, 24.49),
+    (Q4_K, 3, 4096, 4096, 7.71, 7.12), (Q4_K, 5, 4096, 4096, 7.96, 7.50),
+    (Q4_K, 5, 1024, 4096, 7.89, 7.31), (Q4_K, 6, 4096, 4096, 8.05, 8.40),
+    (Q4_K, 8, 4096, 4096, 8.11, 10.04), (Q4_K, 9, 4096, 3584, 7.93, 9.34),
+    (Q4_K, 10, 4096, 2560, 7.76, 9.08), (Q4_K, 12, 4096, 2560, 7.85, 10.17),
+    (Q4_K, 12, 4096, 1280, 8.10, 7.66), (Q4_K, 16, 4096, 768, 7.56, 6.94),
+    (Q4_K, 16, 4096, 2048, 8.61, 11.78), (Q4_K, 16, 1024, 2048, 8.16, 9.33),
+    (Q4_K, 5, 14336, 4096, 15.97, 14.38), (Q4_K, 1, 16384, 4096, 13.66, 14.48),
+    (Q4_K, 4, 5120, 8192, 12.69, 16.16), (Q4_K, 2, 5120, 14336, 16.65, 23.44),
+    (Q4_K, 16, 20480, 2048, 13.37, 14.79), (Q4_K, 8, 28672, 2048, 14.86, 13.79),
+    (Q6_K, 5, 1024, 4096, 10.45, 8.36), (Q6_K, 8, 4096, 4096, 10.55, 9.63),
+    (Q6_K, 16, 4096, 2048, 10.30, 8.88), (Q6_K, 4, 5120, 8192, 18.00, 22.28),
+    (Q6_K, 5, 14336, 6144, 27.57, 25.24), (Q6_K, 3, 5120, 6144, 14.03, 16.42),
+    (Q6_K, 5, 28672, 4096, 31.09, 29.57)]
+
+
+@pytest.mark.parametrize("dt,n,rows,cols,staged,registers", SMALL_BATCH)
+def test_small_batch_takes_the_faster_kernel(rules, dt, n, rows, cols, staged, registers):
+    """3%: what two runs of one side differ by."""
+    if rules.in_registers(dt, n, rows, cols):
+        assert registers <= 1.03 * staged
+    else:
+        assert staged <= 1.03 * registers

@@ -1,8 +1,8 @@
 """The register-x small-batch kernel (few tokens, short rows) at its edges: one
 row, ragged 16-row tiles, one to eight tiles per workgroup and a last workgroup
-with fewer, rows of one quad, of less than a round of waves and of several
-passes, 1-16 tokens, y written and accumulated; and the shapes just past its
-line, which take the staged kernel.  Weights round to fp16 and x to fp16
+with fewer, rows of less than a round of waves and of several passes, 1-16
+tokens, y written and accumulated; and the shapes past its line, which take the
+staged kernel.  Weights round to fp16 and x to fp16
 (2^-11 each, products exact in fp32): an output is within 2^-10 (1 + 2^-11)
 sum |w x| of the exact product, plus the fp32 sums' K 2^-24 sum |w x|, plus
 fp16's smallest step (2^-25 absolute per weight and per x)."""
