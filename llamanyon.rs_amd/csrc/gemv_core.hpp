@@ -5,6 +5,7 @@
 // namespace); the two units compile in parallel.
 #pragma once
 
+#include "dispatch.hpp"
 #include "swamp_common.hpp"
 #include "swamp_items.hpp"
 
@@ -790,8 +791,11 @@ __device__ __forceinline__ void read_vec(float4 (&xv)[16], const uint8_t *lds, i
 // squares) is computed by each set for itself.
 // kX32: fp32 x (XFrag32, the reference's arithmetic); else x rounded to
 // fp16 (XFrag, dot2 arithmetic).
+// kProduct: a SwiGLU prologue forms its product while staging (Product), else
+// gate and up are both staged and every set multiplies its own items
+// (swiglu_product_staged says which).
 template <int DT, int kPPT, int kRows, int kWaves, bool kMulti, int kPro, bool kX32,
-          int kSets = 1>
+          int kSets = 1, bool kProduct = true>
 __global__ void __launch_bounds__(64 * kWaves * kSets)
     gemv_kernel(MatSet ms, const float *__restrict__ x, Pro pro, int ipr, size_t row_bytes,
                 int n_tiles) {
@@ -838,7 +842,8 @@ __global__ void __launch_bounds__(64 * kWaves * kSets)
   constexpr bool kStage = kPPT == 1;  // x through LDS (item count <= 64 kWaves)
   constexpr bool kSwi = kPro == kProSwiGLU || kPro == kProSwiGLUAcc;
   static_assert(kStage || !kSwi, "SwiGLU: one item per lane");
-  constexpr bool kTwo = kStage && kPro == kProRmsNorm && kWaves <= 4;  // both vectors at once
+  constexpr bool kProd = kSwi && kProduct;
+  constexpr bool kTwo = kStage && kPro != kProNone && !kProd && kWaves <= 4;  // both at once
   constexpr int kRegion = kWaves * 16384;
   __shared__ __align__(16) uint8_t xlds[kStage ? (kTwo ? 2 : 1) * kRegion : 16];
   // waves of the workgroup and this wave's index among them (x staging)
@@ -846,8 +851,8 @@ __global__ void __launch_bounds__(64 * kWaves * kSets)
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)), lane = tid & 63;
   float4 x4[kPPT][16];
   [[maybe_unused]] float4 v4[kPPT][16];  // prologue operand (w_norm or up)
-  [[maybe_unused]] Product<DT, kWgWaves, kSwi ? 16 / kSets : 1> prod;
-  if constexpr (kSwi) {
+  [[maybe_unused]] Product<DT, kWgWaves, kProd ? 16 / kSets : 1> prod;
+  if constexpr (kProd) {
     prod.load(x, pro.x2, ipr, wave, lane);
   } else if constexpr (kStage) {
     stage_vec<DT, kWgWaves>(xlds, x, ipr, wave, lane);
@@ -866,7 +871,7 @@ __global__ void __launch_bounds__(64 * kWaves * kSets)
   // keep every load of the tile ahead of the arithmetic (the scheduler would
   // otherwise sink them into registers freed by the current tile)
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (kSwi) {
+  if constexpr (kProd) {
     prod.store(xlds, wave, lane);  // waits for gate and up, not for the tile
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     st.mark(1);
@@ -888,6 +893,15 @@ __global__ void __launch_bounds__(64 * kWaves * kSets)
       stage_vec<DT, kWgWaves>(xlds, pro.x2, ipr, wave, lane);
       asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
       read_vec(v4[0], xlds, item[0]);
+    }
+  }
+  if constexpr (kSwi && !kProd) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      float4 &g = x4[0][i];
+      const float4 u = v4[0][i];
+      g = make_float4(swamp::silu_mul(g.x, u.x), swamp::silu_mul(g.y, u.y),
+                      swamp::silu_mul(g.z, u.z), swamp::silu_mul(g.w, u.w));
     }
   }
   // RMSNorm: W ((x * inv_rms) * w) = inv_rms * (W (x * w)), so the fragment
@@ -1002,7 +1016,8 @@ const Tuning &tuning() {
   return t;
 }
 
-template <int DT, int kPPT, int kRows, int kWaves, int kPro, bool kX32, int kSets = 1>
+template <int DT, int kPPT, int kRows, int kWaves, int kPro, bool kX32, int kSets = 1,
+          bool kProduct = true>
 int launch_items(const MatSet &ms, const float *x, const Pro &pro, int n_cols, hipStream_t s) {
   const int ipr = n_cols / 64;
   if (ipr > kPPT * 64 * kWaves) return SWAMP_ESHAPE;
@@ -1014,12 +1029,12 @@ int launch_items(const MatSet &ms, const float *x, const Pro &pro, int n_cols, h
   if (grid < 1) return SWAMP_OK;
   constexpr int kThreads = 64 * kWaves * kSets;
   if (ms.n == 1)
-    gemv_kernel<DT, kPPT, kRows, kWaves, false, kPro, kX32, kSets>
+    gemv_kernel<DT, kPPT, kRows, kWaves, false, kPro, kX32, kSets, kProduct>
         <<<grid, kThreads, 0, s>>>(ms, x, pro, ipr, swamp::row_bytes(DT, n_cols), n_tiles);
   else if constexpr (kPro == kProSwiGLU || kPro == kProSwiGLUAcc)
     return SWAMP_EINVAL;  // single matrix only
   else
-    gemv_kernel<DT, kPPT, kRows, kWaves, true, kPro, kX32, kSets>
+    gemv_kernel<DT, kPPT, kRows, kWaves, true, kPro, kX32, kSets, kProduct>
         <<<grid, kThreads, 0, s>>>(ms, x, pro, ipr, swamp::row_bytes(DT, n_cols), n_tiles);
   return hipGetLastError() == hipSuccess ? SWAMP_OK : SWAMP_ELAUNCH;
 }
@@ -1116,6 +1131,12 @@ int launch_rows(const MatSet &ms, const float *x, const Pro &pro, int n_cols, hi
       return launch_items<DT, 1, kRows, 1, kPro, kX32>(ms, x, pro, n_cols, s);
     }
     if (ipr <= 128) {
+      if constexpr ((kPro == kProSwiGLU || kPro == kProSwiGLUAcc) &&
+                    (DT == SWAMP_Q8_0 || DT == SWAMP_Q6_K)) {
+        if (ms.sets && ms.wpc >= 8 &&
+            !swamp::swiglu_product_staged(DT, ms.rows[0], n_cols, swamp::device_info().num_cus))
+          return launch_items<DT, 1, kRows, 2, kPro, kX32, 2, false>(ms, x, pro, n_cols, s);
+      }
       if (ms.sets && ms.wpc >= 8) return launch_items<DT, 1, kRows, 2, kPro, kX32, 2>(ms, x, pro, n_cols, s);
       return launch_items<DT, 1, kRows, 2, kPro, kX32>(ms, x, pro, n_cols, s);
     }

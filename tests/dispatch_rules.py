@@ -24,6 +24,9 @@ int dequantize_once(unsigned dt, int m, int rows, int cols, int cus) {
 int in_registers(unsigned dt, int n, int rows, int cols, int cus) {
   return swamp::small_batch_in_registers(dt, n, rows, cols, cus);
 }
+int product_staged(unsigned dt, int rows, int cols, int cus) {
+  return swamp::swiglu_product_staged(dt, rows, cols, cus);
+}
 }
 """
 
@@ -49,3 +52,6 @@ class Rules:
 
     def in_registers(self, dt, n, rows, cols, cus=CUS):
         return bool(self.lib.in_registers(dt, n, rows, cols, cus))
+
+    def product_staged(self, dt, rows, cols, cus=CUS):
+        return bool(self.lib.product_staged(dt, rows, cols, cus))

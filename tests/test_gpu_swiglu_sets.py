@@ -1,7 +1,7 @@
-"""The SwiGLU GEMV with two row sets of four waves per workgroup (rows of 8193
+"""The SwiGLU GEMV with two row sets per workgroup, of four waves (rows of 8193
 to 16384 weights) where its second set runs out of tiles: one row, an odd number
-of tiles, one tile more than a round, the smallest Q6_K matrix that takes it;
-written and accumulated.  h = silu(gate) up is formed with hardware exp2 and
+of tiles, one tile more than a round; and of two waves (rows of 4097 to 8192)
+on both sides of the line between its two prologues; written and accumulated.  h = silu(gate) up is formed with hardware exp2 and
 reciprocal (about 1 ulp each) and y in fp32, so an output is within
 (cols + 16) 2^-24 sum |w h| of the exact sum, and the add rounds once more."""
 import numpy as np
@@ -14,7 +14,8 @@ Q4_0, Q8_0, Q4_K, Q6_K = 2, 8, 12, 14
 
 @pytest.mark.parametrize("dtype", [Q4_0, Q8_0, Q4_K, Q6_K])
 @pytest.mark.parametrize("rows,cols", [(1, 8704), (3, 16384), (513, 9216), (1027, 11264),
-                                       (3073, 8704), (4099, 14336)])
+                                       (3073, 8704), (4099, 14336), (1, 4608), (2048, 8192),
+                                       (2049, 4608), (2051, 7680), (4099, 8192)])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_swiglu_two_sets(pkg, orc, dtype, rows, cols, accumulate):
     torch = pytest.importorskip("torch")
