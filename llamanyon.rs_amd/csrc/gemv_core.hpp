@@ -1144,10 +1144,10 @@ int launch_rows(const MatSet &ms, const float *x, const Pro &pro, int n_cols, hi
     // and up and makes their product twice per CU (115 KB and 14336
     // exponentials for an 8B down projection).  us, two sets / one: 4096 x
     // 14336 Q6_K 15.8 / 17.0, Q4_K 10.7 / 12.0, Q4_0 9.8 / 11.2, Q8_0 14.1 /
-    // 16.5; 8192 x 14336 Q4_K 17.1 / 18.0; 2560 x 9216 Q4_K 8.7 / 9.0, but Q6_K
-    // 11.8 / 11.7: too few rows for its single-row tiles.
+    // 16.5; 8192 x 14336 Q4_K 17.1 / 18.0; Q6_K 1024 x 14336 8.5 / 10.0, 2304 to
+    // 2560 rows the same within 2%.
     if constexpr (kPro == kProSwiGLU || kPro == kProSwiGLUAcc) {
-      if (ipr <= 256 && ms.sets && ms.wpc >= 8 && (DT != SWAMP_Q6_K || ms.rows[0] >= 3072))
+      if (ipr <= 256 && ms.sets && ms.wpc >= 8)
         return launch_items<DT, 1, kRows, 4, kPro, kX32, 2>(ms, x, pro, n_cols, s);
     }
     if (ipr <= 256) return launch_items<DT, 1, kRows, 4, kPro, kX32>(ms, x, pro, n_cols, s);
