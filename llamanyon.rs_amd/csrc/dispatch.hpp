@@ -200,14 +200,19 @@ inline bool small_batch_in_registers(uint32_t dtype, int n_tok, int n_rows, int 
 // every row set.  The product is formed sooner, but with Q8_0 and Q6_K rows of
 // 4097 to 8192 weights (two waves per row) matrices of more than one tile per
 // row set measured slower behind it (the tile loop is the same code; in the
-// other form each wave reaches it at its own time).  us, both staged / product: Q8_0 1536 x 8192 7.1 / 6.2, 2048 8.0 / 7.7, 2100
-// 8.2 / 8.6, 6144 13.2 / 14.6, 8192 15.6 / 17.1; Q6_K 1900 x 5632 8.4 / 7.2,
-// 2304 8.7 / 8.9, 4096 x 8192 11.3 / 12.8; Q4_K 4096 x 8192 8.9 / 8.2, 8192 x
-// 8192 12.2 / 12.0.  Other row lengths gain everywhere: Q8_0 8192 x 4096
-// 0.92 of the time, 8192 x 14336 0.91, Q6_K 8192 x 8704 0.80.
-inline bool swiglu_product_staged(uint32_t dtype, int n_rows, int n_cols, int cus) {
-  const bool nibbles = dtype == SWAMP_Q4_0 || dtype == SWAMP_Q4_K;
-  return nibbles || n_cols <= 4096 || n_cols > 8192 || n_rows <= 8 * cus;
+// other form each wave reaches it at its own time): Q8_0 beyond 8 rows of 8192
+// weights per CU, Q6_K beyond 8 rows per CU, 12 when it adds to y.  us, both staged /
+// product: Q8_0 2048 x 8192 8.0 / 7.7, 2100 x 8192 8.2 / 8.6, 2816 x 5632 8.1 /
+// 8.0, 5120 x 5632 9.6 / 10.5, 6144 x 8192 13.2 / 14.6, 8192 15.6 / 17.1; Q6_K
+// 1900 x 5632 8.4 / 7.2, 2304 8.7 / 8.9, 4096 x 8192 11.3 / 12.8, added 2560 x
+// 8192 10.1 / 9.3, 4096 12.2 / 12.9; Q4_K 4096 x 8192 8.9 / 8.2, 8192 x 8192 12.2 /
+// 12.0.  Other row lengths gain everywhere: Q8_0 8192 x 4096 10.4 / 9.6, 8192 x
+// 14336 27.3 / 24.8, Q6_K 8192 x 8704 31.3 / 24.9.
+inline bool swiglu_product_staged(uint32_t dtype, int n_rows, int n_cols, bool accumulate,
+                                  int cus) {
+  if (dtype == SWAMP_Q4_0 || dtype == SWAMP_Q4_K || n_cols <= 4096 || n_cols > 8192) return true;
+  if (dtype == SWAMP_Q8_0) return long(n_rows) * n_cols <= 8L * 8192 * cus;
+  return n_rows <= (accumulate ? 12 : 8) * cus;
 }
 
 }  // namespace swamp

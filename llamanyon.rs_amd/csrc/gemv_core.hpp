@@ -1134,7 +1134,8 @@ int launch_rows(const MatSet &ms, const float *x, const Pro &pro, int n_cols, hi
       if constexpr ((kPro == kProSwiGLU || kPro == kProSwiGLUAcc) &&
                     (DT == SWAMP_Q8_0 || DT == SWAMP_Q6_K)) {
         if (ms.sets && ms.wpc >= 8 &&
-            !swamp::swiglu_product_staged(DT, ms.rows[0], n_cols, swamp::device_info().num_cus))
+            !swamp::swiglu_product_staged(DT, ms.rows[0], n_cols, kPro == kProSwiGLUAcc,
+                                          swamp::device_info().num_cus))
           return launch_items<DT, 1, kRows, 2, kPro, kX32, 2, false>(ms, x, pro, n_cols, s);
       }
       if (ms.sets && ms.wpc >= 8) return launch_items<DT, 1, kRows, 2, kPro, kX32, 2>(ms, x, pro, n_cols, s);

@@ -74,22 +74,25 @@ def test_small_batch_takes_the_faster_kernel(rules, dt, n, rows, cols, staged, r
         assert staged <= 1.03 * registers
 
 
-# (dtype, rows, weights per row, us both vectors staged, us product staged)
+# (dtype, rows, weights per row, added to y, us both vectors staged, us product staged)
 SWIGLU = [
-    (Q4_0, 2560, 8192, 7.49, 6.90), (Q4_0, 14336, 8192, 15.52, 15.26),
-    (Q4_K, 4096, 5632, 8.64, 7.64), (Q4_K, 8192, 8192, 12.13, 11.96),
-    (Q8_0, 1536, 8192, 7.08, 6.24), (Q8_0, 2048, 8192, 7.99, 7.70),
-    (Q8_0, 2100, 8192, 8.24, 8.59), (Q8_0, 5120, 5632, 9.55, 10.53),
-    (Q8_0, 6144, 8192, 13.17, 14.55), (Q8_0, 8192, 8192, 15.56, 17.02),
-    (Q8_0, 8192, 4096, 10.40, 9.56), (Q8_0, 14336, 16384, 46.47, 43.60),
-    (Q6_K, 1900, 5632, 8.43, 7.19), (Q6_K, 4096, 8192, 11.29, 12.83),
-    (Q6_K, 8192, 5632, 15.08, 15.99), (Q6_K, 8192, 8192, 16.54, 17.75),
-    (Q6_K, 8192, 8704, 31.34, 24.93)]
+    (Q4_0, 2560, 8192, False, 7.49, 6.90), (Q4_0, 14336, 8192, False, 15.52, 15.26),
+    (Q4_K, 4096, 5632, False, 8.64, 7.64), (Q4_K, 8192, 8192, False, 12.13, 11.96),
+    (Q8_0, 1536, 8192, False, 7.08, 6.24), (Q8_0, 2048, 8192, False, 7.99, 7.70),
+    (Q8_0, 2304, 5632, False, 8.05, 7.63), (Q8_0, 3072, 4608, False, 7.98, 7.61),
+    (Q8_0, 2304, 8192, False, 8.43, 8.81), (Q8_0, 2560, 5632, True, 8.62, 8.09),
+    (Q8_0, 5120, 5632, False, 9.55, 10.53), (Q8_0, 6144, 8192, False, 13.17, 14.55),
+    (Q8_0, 8192, 8192, False, 15.56, 17.02), (Q8_0, 8192, 4096, False, 10.40, 9.56),
+    (Q8_0, 14336, 16384, False, 46.47, 43.60), (Q6_K, 1900, 5632, False, 8.43, 7.19),
+    (Q6_K, 2560, 8192, True, 10.06, 9.29), (Q6_K, 2560, 5632, True, 9.32, 8.89),
+    (Q6_K, 4096, 8192, True, 12.22, 12.91), (Q6_K, 4096, 8192, False, 11.29, 12.83),
+    (Q6_K, 8192, 5632, False, 15.08, 15.99), (Q6_K, 8192, 8192, False, 16.54, 17.75),
+    (Q6_K, 8192, 8704, False, 31.34, 24.93)]
 
 
-@pytest.mark.parametrize("dt,rows,cols,both,product", SWIGLU)
-def test_swiglu_takes_the_faster_prologue(rules, dt, rows, cols, both, product):
-    if rules.product_staged(dt, rows, cols):
+@pytest.mark.parametrize("dt,rows,cols,add,both,product", SWIGLU)
+def test_swiglu_takes_the_faster_prologue(rules, dt, rows, cols, add, both, product):
+    if rules.product_staged(dt, rows, cols, add):
         assert product <= 1.03 * both
     else:
         assert both <= 1.03 * product
