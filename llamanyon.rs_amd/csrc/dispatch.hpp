@@ -28,14 +28,21 @@ constexpr int kGemmTokens = 256, kGemmRows = 256, kGemmK = 64;
 // Split pieces write partial tiles to scratch, summed in piece order by a
 // second kernel (deterministic).  Without scratch the pieces add into
 // zeroed y with float atomics (and kSplit takes halves).
-// The kSplit estimate: measured time of a K step of one tile while a round is
-// full (below; 0.7 of it when few are in flight), 6 us to fill a whole tile's
-// stages and store it, and the partial sums at 6 TB/s, written (partly behind other tiles), read, y written.  It replaced a
-// choice of full tiles or halves in at most 4 pieces, both halves of a tile
-// counted: 100 tokens x 6144 x 4096 Q4_K 31.3 -> 25.4 us (halves, 8 pieces),
-// 150 x 4096 x 14336 57.0 -> 45.1, 70 x 4096 x 4096 27.0 -> 20.3, 256 x 4096 x
-// 4096 29.8 -> 26.1 (quarters), 300 x 6144 x 4096 47.0 -> 35.7 (halves), 120 x
-// 3000 x 28672 88.1 -> 54.5.
+// The kSplit estimate is fitted to the measured times of every part size and
+// piece count of 3052 shapes (65 to 2048 tokens, 1024 to 28672 rows, 1024 to 28672
+// weights, all formats; it meets those near the best of their shape within 3%
+// rms): 13 us to fill a whole tile's stages and store it, the K steps below
+// while a round is full (0.78 of a step when few tiles are in flight), 5.7 us for
+// the second kernel and its partial sums, written and read, at 2.3 TB/s per
+// piece.  The choice is within 0.5% of the best on average, 16% at worst.  An
+// estimate from single shapes (2.04 us a step, 2 us for the second kernel) had
+// split where it does not pay and taken halves where whole tiles in two pieces
+// are faster: us, that choice / this one, 256 tokens x 4096 x 1024 Q4_0 19.2 /
+// 15.4 (quarters, 2 pieces / 1), 300 x 14336 x 5120 Q8_0 109.9 / 90.4 (halves /
+// whole tiles in 2 pieces), 640 x 8192 x 5120 Q8_0 107.9 / 87.3.  The choice of
+// full tiles or halves in at most 4 pieces, both halves of a tile counted, that
+// was there before either: 100 x 6144 x 4096 Q4_K 31.3, now 25.4, 300 x 6144 x
+// 4096 47.0, now 35.7, 120 x 3000 x 28672 88.1, now 54.5.
 struct GemmPlan {
   enum Kind { kSmall, kSplit, kRounds } kind;
   int parts;      // kSplit: tiles run whole (1), as halves (2) or quarters (4)
@@ -45,11 +52,12 @@ struct GemmPlan {
   size_t part_bytes;          // scratch for the pieces' partial sums
 };
 
-// us of one K step of a whole tile, a half, a quarter, in a full round.
+// us of one K step of a whole tile, a half, a quarter, in a full round (fitted
+// with the rest of the estimate, above).
 constexpr double gemm_step_us(uint32_t dt, int parts) {
-  return dt == SWAMP_Q6_K   ? (parts == 1 ? 2.65 : 1.68)
-         : dt == SWAMP_Q8_0 ? (parts == 1 ? 2.25 : parts == 2 ? 1.40 : 1.11)
-                            : (parts == 1 ? 2.04 : parts == 2 ? 1.17 : 0.82);
+  return dt == SWAMP_Q6_K   ? (parts == 1 ? 1.96 : 1.58)
+         : dt == SWAMP_Q8_0 ? (parts == 1 ? 1.66 : parts == 2 ? 1.28 : 1.10)
+                            : (parts == 1 ? 1.42 : parts == 2 ? 0.98 : 0.78);
 }
 
 inline GemmPlan plan_gemm_bf16(uint32_t dt, int m, int n_rows, int n_cols, int cus) {
@@ -98,8 +106,8 @@ inline GemmPlan plan_gemm_bf16(uint32_t dt, int m, int n_rows, int n_cols, int c
         if (part > cap) break;
         const double fill = double(units) * pieces / cus, rounds = std::ceil(fill);
         double t =
-            6.0 / parts + kps * gemm_step_us(dt, parts) * rounds * (0.7 + 0.3 * fill / rounds);
-        if (pieces > 1) t += 2.0 + (1.3 * pieces + 1.0) * double(mn) * 4.0 / 6e6;
+            13.0 / parts + kps * gemm_step_us(dt, parts) * rounds * (0.78 + 0.22 * fill / rounds);
+        if (pieces > 1) t += 5.7 + 1.75 * pieces * double(mn) * 4.0 / 6e6;
         if (best == 0 || t < best) {
           best = t;
           p.parts = parts;

@@ -5,7 +5,7 @@ import types
 
 import pytest
 
-from dispatch_rules import CUS, REPO, Q4_0, Q4_K, Q6_K, Q8_0, Rules
+from dispatch_rules import CUS, REPO, SPLIT, Q4_0, Q4_K, Q6_K, Q8_0, Rules
 
 
 @pytest.fixture(scope="session")
@@ -96,3 +96,42 @@ def test_swiglu_takes_the_faster_prologue(rules, dt, rows, cols, add, both, prod
         assert product <= 1.03 * both
     else:
         assert both <= 1.03 * product
+
+
+# (dtype, tokens, rows, weights per row, us of each (parts of a tile, K pieces)
+# within 1.3 times the fastest)
+PLANS = [
+    (Q4_0, 256, 4096, 1024, {(4, 1): 15.4, (4, 2): 19.2}),
+    (Q4_0, 640, 10240, 14336, {(1, 2): 206.6, (2, 1): 238.7}),
+    (Q4_0, 300, 14336, 14336, {(1, 2): 193.0, (2, 1): 220.7}),
+    (Q4_0, 100, 6144, 4096, {(2, 4): 29.5, (2, 5): 29.3, (2, 6): 27.8, (2, 7): 26.9, (2, 8):
+     27.2, (4, 2): 30.6, (4, 3): 26.7, (4, 4): 26.2, (4, 5): 24.6}),
+    (Q4_0, 512, 6144, 4096, {(1, 3): 56.9, (1, 4): 52.8, (1, 5): 54.0, (2, 1): 58.4, (2, 2):
+     46.5, (4, 1): 47.6}),
+    (Q8_0, 300, 14336, 5120, {(1, 2): 90.4, (2, 1): 109.9}),
+    (Q8_0, 640, 8192, 5120, {(1, 2): 87.3, (2, 1): 107.9}),
+    (Q8_0, 300, 6144, 28672, {(1, 4): 205.2, (1, 5): 180.3, (2, 3): 206.2}),
+    (Q8_0, 777, 2048, 1024, {(2, 1): 23.1, (4, 1): 19.3, (4, 2): 23.8}),
+    (Q8_0, 128, 4096, 4096, {(2, 5): 30.7, (2, 6): 29.7, (2, 7): 28.9, (2, 8): 28.4, (4, 4):
+     29.1, (4, 5): 26.9, (4, 6): 25.3, (4, 7): 24.9, (4, 8): 24.5}),
+    (Q4_K, 512, 2048, 1024, {(4, 1): 15.6, (4, 2): 19.5}),
+    (Q4_K, 150, 6144, 1024, {(2, 1): 20.9, (4, 1): 16.1, (4, 2): 19.1}),
+    (Q4_K, 150, 6144, 4096, {(1, 6): 38.2, (1, 8): 35.4, (2, 3): 36.5, (2, 4): 31.4, (4, 2):
+     32.8, (4, 3): 29.9}),
+    (Q4_K, 2048, 4096, 14336, {(1, 2): 229.8, (2, 1): 247.2}),
+    (Q4_K, 65, 1024, 14336, {(2, 7): 36.0, (2, 8): 32.8, (4, 6): 34.5, (4, 7): 30.2, (4, 8):
+     27.9}),
+    (Q6_K, 300, 6144, 28672, {(1, 4): 235.3, (1, 5): 205.0, (2, 3): 246.3}),
+    (Q6_K, 640, 4096, 1024, {(2, 1): 28.8, (2, 2): 34.4}),
+    (Q6_K, 777, 4096, 14336, {(1, 3): 164.0, (1, 4): 141.7, (2, 2): 177.5}),
+    (Q6_K, 512, 4096, 4096, {(1, 4): 57.3, (1, 6): 55.1, (1, 8): 54.9, (2, 2): 59.6, (2, 3):
+     51.9, (2, 4): 46.0})]
+
+
+@pytest.mark.parametrize("dt,m,rows,cols,us", PLANS)
+def test_gemm_plan_is_near_the_fastest(rules, dt, m, rows, cols, us):
+    """5%: what two runs of one plan differ by at these sizes (they are bound
+    by power, so the clock moves with what ran before)."""
+    kind, parts, pieces, _, _ = rules.plan(dt, m, rows, cols)
+    assert kind == SPLIT
+    assert us.get((parts, pieces), 1e9) <= 1.05 * min(us.values()), (parts, pieces)
