@@ -384,18 +384,23 @@ def layer_lines(pkg, torch, stream, lib, shapes, sigma, n_toks, seed):
 
 def gemm_route(torch, dtype_q6k, m, rows, k, x_name):
     """Which of the library's kernels a swamp_qgemm call runs, by the rule
-    of swamp_gemm_dq_route (csrc/gemm_dq.hip): bf16 x takes the
+    of gemm_dequantize_once (csrc/dispatch.hpp): bf16 x takes the
     dequantize-once route (blocks_to_bf16 + gemm_bb) for Q6_K except from 65
     tokens where its fused kernel is faster, and from 1024 tokens for shapes
-    whose 256 x 256 tiles fill more than half but not all of the CUs; else the fused dequant GEMM (gemm_bf16_kernel).  Q8_0 x runs
+    whose 256 x 256 tiles fill more than half but not all of the CUs; else the
+    fused dequant GEMM (gemm_bf16_kernel).  Q8_0 x runs
     the int8 GEMM."""
     if x_name != "bf16":
         return "gemm_i8 (int8 MFMA)"
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     tiles = ((m + 255) // 256) * ((rows + 255) // 256)
     if dtype_q6k:
-        dq = not (m > 64 and k % 512 == 0 and 16 * tiles >= cus and
-                  (m <= 512 or (2 * tiles <= cus and k >= 8192)))
+        if m <= 64 or k % 512:
+            dq = True
+        elif m <= 512:
+            dq = (16 if m <= 256 or k > 8192 else 10) * tiles < cus
+        else:
+            dq = k <= 8192 or 2 * tiles > cus or (16 if k >= 20480 else 8) * tiles < cus
     else:
         dq = m >= 1024 and k >= 1024 and 2 * tiles > cus and tiles < cus
     if dq:

@@ -223,8 +223,9 @@ SWAMP_API int swamp_qgemv_batched(uint32_t dtype, const void *d_w, size_t w_len,
  * weight); when the tiles do not fill the GPU, K is split across
  * workgroups whose partial tiles go to scratch and are summed in piece
  * order by a second kernel (deterministic).  For Q6_K of at most 64 tokens,
- * of rows of an odd number of blocks, or of many tokens (more than 512, when
- * the rows are short or the tiles fill the GPU), and otherwise
+ * of rows of an odd number of blocks, of too few tiles to split, or of more
+ * than 512 tokens on rows of up to 8192 weights or past half a round of tiles,
+ * and for the other formats
  * from 1024 tokens when 256 x 256 tiles would fill more than half but not
  * all of the CUs (e.g. 2048 tokens x 6144 rows), the weights are instead
  * dequantized once per call to bf16 in scratch (row chunks of at most

@@ -132,16 +132,23 @@ inline bool gemm_dequantize_once(uint32_t dtype, int m, int n_rows, int n_cols, 
   const long tiles = long((m + 255) / 256) * long((n_rows + 255) / 256);
   if (dtype == SWAMP_Q6_K) {
     // Q6_K's fused dequantization takes twice the vector work of the others
-    // per matrix instruction; this route instead writes and re-reads 2 bytes
-    // per weight.  Fused where that traffic counts most: few tokens, or long
-    // rows whose tiles split along K -- but not where too few tiles are left
-    // to split.  us, fused / this route: 512 x 28672 x 4096 158 / 182, 600
-    // 247 / 247, 1000 298 / 289; 512 x 6144 x 4096 66 / 66, 1000 103 / 88;
-    // 777 x 4096 x 14336 150 / 187, 1500 254 / 295, 2048 286 / 312; 200 x
-    // 3000 x 5120 (12 tiles) 40 / 32, 70 x 2048 x 14336 (8 tiles) 57 / 46.
+    // per matrix instruction, once per token tile; this route instead writes
+    // and re-reads 2 bytes per weight, once.  Fused where that traffic counts
+    // most -- one token tile, or two, or long rows whose tiles split along K --
+    // and enough tiles are left to split.  Timed on 2146 shapes; us, fused /
+    // this route.  One token tile: 65 x 4096 x 4096 25.9 / 30.1, 128 x 28672 x
+    // 4096 74 / 141, 256 x 4096 x 14336 71 / 82, but with 8 or 4 tiles 65 x 2048 x
+    // 14336 53 / 46, 256 x 1024 x 8192 36 / 33.  Two: 512 x 28672 x 4096 149 /
+    // 183, 350 x 3584 x 6144 45 / 52, 512 x 4096 x 4096 46 / 46, 300 x 14336 x
+    // 4096 88 / 86, but 512 x 3000 x 8192 (24 tiles) 65 / 59, 512 x 2048 x 1024
+    // 26 / 22; over 8192 weights 16 tiles do: 450 x 3584 x 10240 71 / 79.  More:
+    // 777 x 4096 x 14336 143 / 158, 700 x 7168 x 10240 153 / 191, 777 x 2048 x
+    // 28672 150 / 164, but 1300 x 4096 x 8192 141 / 117, 1000 x 6144 x 4096 102 /
+    // 75, and past half a round 1300 x 6144 x 14336 394 / 339.
     if (!q6k_gemm_fusable(m, n_cols)) return true;
-    const bool fused = 16 * tiles >= cus && (m <= 512 || (2 * tiles <= cus && n_cols >= 8192));
-    return !fused;
+    if (m <= 256) return 16 * tiles < cus;
+    if (m <= 512) return (n_cols > 8192 ? 16 : 10) * tiles < cus;
+    return n_cols <= 8192 || 2 * tiles > cus || (n_cols >= 20480 ? 16 : 8) * tiles < cus;
   }
   // The fused kernel reads 0.56-1.06 bytes per weight per tile, the plain
   // bf16 GEMM 2 (its loads from L2 bound it, not the dequantization), so the

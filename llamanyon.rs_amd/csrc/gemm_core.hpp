@@ -32,10 +32,9 @@
 //    supplies 2^9): low nibbles masked in place, high ones shifted down.
 //    Q6_K codes are assembled to bytes, converted one by one and multiplied
 //    by their group's scale: 5 vector instructions per MFMA against 2.75, so
-//    a step takes 2.4 us where the nibble formats take 2.0 (777 tokens x
-//    4096 rows x 14336: 151 us against Q4_K's 128; 187 us before, with the
-//    weights dequantized to memory first).  gemm_dq.hip draws the line
-//    between the two.
+//    a call takes up to 1.4 times the nibble formats' (777 tokens x 4096 rows x
+//    14336: 143 us against Q4_K's 125; 158 with the weights dequantized to
+//    memory first).  dispatch.hpp draws the line between the two.
 //  * Tile order: groups of 4 token tiles, consecutive tiles walking the
 //    weight columns of a group; workgroup ids are remapped so each XCD
 //    (ids i, i+8, ...) runs a contiguous run of that order.  A round of an

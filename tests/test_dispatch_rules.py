@@ -30,7 +30,7 @@ def test_bench_route_labels_follow_the_rule(rules, bench):
     for dt in (Q4_0, Q8_0, Q4_K, Q6_K):
         for m in (1, 64, 65, 128, 129, 256, 257, 512, 513, 777, 1000, 1023, 1024, 1025, 2048, 4096):
             for rows in (1, 256, 1000, 2048, 4096, 4097, 6144, 8192, 14336, 28672, 128256):
-                for cols in (512, 768, 1024, 4096, 4352, 7680, 8192, 14336, 28672):
+                for cols in (512, 768, 1024, 4096, 4352, 8192, 8704, 14336, 19968, 20480):
                     want = rules.dequantize_once(dt, m, rows, cols)
                     label = bench.gemm_route(gpu, dt == Q6_K, m, rows, cols, "bf16")
                     assert label.startswith("dequantize-once") == want, (dt, m, rows, cols, label)
@@ -135,3 +135,25 @@ def test_gemm_plan_is_near_the_fastest(rules, dt, m, rows, cols, us):
     kind, parts, pieces, _, _ = rules.plan(dt, m, rows, cols)
     assert kind == SPLIT
     assert us.get((parts, pieces), 1e9) <= 1.05 * min(us.values()), (parts, pieces)
+
+
+# (tokens, rows, weights per row, us fused, us dequantized once), Q6_K
+Q6K_ROUTES = [
+    (65, 4096, 4096, 25.9, 30.1), (65, 2048, 14336, 53.4, 46.5), (128, 28672, 4096, 74.2, 141.1),
+    (256, 4096, 14336, 70.9, 81.8), (256, 1024, 8192, 36.0, 32.5), (300, 3000, 28672, 123.3, 163.5),
+    (350, 3584, 6144, 44.7, 52.0), (400, 2048, 2048, 29.2, 25.4), (450, 3584, 10240, 71.2, 78.9),
+    (512, 2048, 1024, 26.2, 22.1), (512, 3000, 8192, 64.6, 59.3), (512, 4096, 4096, 46.1, 46.4),
+    (512, 28672, 4096, 148.6, 183.4), (512, 128256, 4096, 630.0, 769.2),
+    (520, 6144, 14336, 167.9, 265.4), (700, 7168, 10240, 153.0, 190.6),
+    (777, 2048, 28672, 150.2, 164.5), (777, 4096, 14336, 143.2, 157.9),
+    (1000, 2048, 8192, 70.4, 61.0), (1000, 6144, 4096, 102.2, 74.6), (1300, 4096, 8192, 140.6, 117.1),
+    (1300, 6144, 14336, 394.4, 338.7), (1700, 1024, 8192, 66.2, 55.9), (1700, 1024, 28672, 149.5, 161.3),
+    (2048, 3000, 8192, 145.1, 121.5), (2048, 4096, 8192, 172.7, 152.6)]
+
+
+@pytest.mark.parametrize("m,rows,cols,fused,once", Q6K_ROUTES)
+def test_q6k_gemm_takes_the_faster_route(rules, m, rows, cols, fused, once):
+    if rules.dequantize_once(Q6_K, m, rows, cols):
+        assert once <= 1.03 * fused
+    else:
+        assert fused <= 1.03 * once
