@@ -231,9 +231,10 @@ SWAMP_API int swamp_qgemv_batched(uint32_t dtype, const void *d_w, size_t w_len,
  * dequantized once per call to bf16 in scratch (row chunks of at most
  * 512 MB; the same bf16 values) and each chunk runs through this library's
  * plain bf16 x bf16 -> fp32 MFMA GEMM, whose 192- and 128-row tiles fill
- * the CUs; when that scratch cannot be had the fused kernel runs (Q6_K, also
- * for the partial tiles of its fused kernel: SWAMP_EWORKSPACE).  Both routes sum in a fixed order: repeated calls
- * give the same bits. */
+ * the CUs; when that scratch cannot be had the fused kernel runs (Q6_K of at
+ * most 64 tokens or of rows of an odd number of blocks: SWAMP_EWORKSPACE).
+ * With their scratch both routes sum in a fixed order: repeated calls give the
+ * same bits. */
 SWAMP_API int swamp_qgemm(uint32_t dtype, const void *d_w, size_t w_len,
                 const void *d_x, uint32_t x_type, float *d_y, int m,
                 int n_rows, int n_cols, void *stream);
@@ -256,7 +257,12 @@ SWAMP_API int swamp_qgemm(uint32_t dtype, const void *d_w, size_t w_len,
  * one host thread at a time: two threads calling on the same stream (the
  * null stream included) at once race on its buffer.
  *   swamp_qgemv_batched_workspace / swamp_qgemm_workspace: the scratch
- *     bytes such a call takes (0: none);
+ *     bytes such a call takes (0: none; Q6_K GEMM: at least those of its
+ *     dequantized weights, also where the fused kernel needs less, so that a
+ *     long prompt's report holds the weights of a short one).  They do not
+ *     grow with the token count: a prompt that fills the GPU takes none, a
+ *     shorter one partial sums.  To reserve for calls of several lengths,
+ *     take the largest report of those lengths;
  *   swamp_workspace_reserve: make the stream's buffer at least `bytes`
  *     long now (for example before capturing calls into a graph); 0, or
  *     SWAMP_EWORKSPACE when it cannot be allocated or the stream is being

@@ -403,7 +403,11 @@ int swamp_qgemm(uint32_t dtype, const void *d_w, size_t w_len, const void *d_x, 
   if (int rc = ensure_device(nullptr)) return rc;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (n_cols == 0) return fill_zero(d_y, size_t(m) * size_t(n_rows), s);
-  Scratch sc = stream_scratch(s, swamp_gemm_scratch_bytes(dtype, x_type, m, n_rows, n_cols));
+  const size_t need = swamp_gemm_scratch_bytes(dtype, x_type, m, n_rows, n_cols);
+  Scratch sc = stream_scratch(s, need);
+  // a buffer reserved for the dequantized weights alone (swamp_qgemm_workspace)
+  if (dtype == SWAMP_Q6_K && need > sc.cap)
+    sc = stream_scratch(s, swamp_gemm_dq_scratch_bytes(m, n_rows, n_cols));
   return swamp_launch_gemm(dtype, d_w, d_x, x_type, d_y, m, n_rows, n_cols, sc, s);
 }
 
@@ -442,7 +446,12 @@ size_t swamp_qgemv_batched_workspace(uint32_t dtype, int n_tok, int n_rows, int 
 
 size_t swamp_qgemm_workspace(uint32_t dtype, uint32_t x_type, int m, int n_rows, int n_cols) {
   if (ensure_device(nullptr) != SWAMP_OK) return 0;
-  return swamp_gemm_scratch_bytes(dtype, x_type, m, n_rows, n_cols);
+  const size_t need = swamp_gemm_scratch_bytes(dtype, x_type, m, n_rows, n_cols);
+  // Q6_K prompts of a few tokens run only with their weights dequantized to
+  // scratch: what a long prompt reports holds those too
+  if (dtype == SWAMP_Q6_K && x_type == SWAMP_BF16 && m > 0 && n_rows > 0 && n_cols > 0)
+    return std::max(need, swamp_gemm_dq_scratch_bytes(m, n_rows, n_cols));
+  return need;
 }
 
 int swamp_workspace_reserve(void *stream, size_t bytes) {

@@ -192,17 +192,18 @@ int swamp_launch_gemm(uint32_t dtype, const void *d_w, const void *d_x, uint32_t
   if (size_t(m) * size_t(n_cols) * 2 > size_t(UINT32_MAX)) return SWAMP_ESHAPE;
   // long prompts: dequantize once to bf16 and run a plain bf16 GEMM, when
   // the scratch for it is there (else the fused kernel below)
-  if (swamp_gemm_dq_route(dtype, m, n_rows, n_cols) &&
-      sc.cap - sc.used >= swamp_gemm_dq_scratch_bytes(m, n_rows, n_cols)) {
+  bool once = swamp_gemm_dq_route(dtype, m, n_rows, n_cols);
+  // Q6_K scratch too small for the fused kernel's partial sums may still hold
+  // the weights
+  if (dtype == SWAMP_Q6_K && sc.cap - sc.used < swamp_gemm_q6k_scratch_bytes(m, n_rows, n_cols))
+    once = true;
+  if (once && sc.cap - sc.used >= swamp_gemm_dq_scratch_bytes(m, n_rows, n_cols)) {
     const size_t used = sc.used;
     const int rc = swamp_launch_gemm_dq(dtype, d_w, d_x, d_y, m, n_rows, n_cols, sc, s);
     if (rc != kDqUnavailable) return rc;
     sc.used = used;
   }
-  if (dtype == SWAMP_Q6_K) {
-    if (swamp_gemm_dq_route(dtype, m, n_rows, n_cols)) return SWAMP_EWORKSPACE;
-    return swamp_launch_gemm_q6k(d_w, d_x, d_y, m, n_rows, n_cols, sc, s);
-  }
+  if (dtype == SWAMP_Q6_K) return swamp_launch_gemm_q6k(d_w, d_x, d_y, m, n_rows, n_cols, sc, s);
   const uint8_t *w = static_cast<const uint8_t *>(d_w);
   const uint16_t *x = static_cast<const uint16_t *>(d_x);
   switch (dtype) {

@@ -189,8 +189,9 @@ bool swamp_gemm_dq_route(uint32_t dtype, int m, int n_rows, int n_cols);
 size_t swamp_gemm_dq_scratch_bytes(int m, int n_rows, int n_cols);
 int swamp_launch_gemm_dq(uint32_t dtype, const void *d_w, const void *d_x, float *d_y, int m,
                          int n_rows, int n_cols, swamp::Scratch &sc, hipStream_t s);
-// The fused GEMM of Q6_K weights (gemm_q6k.hip): SWAMP_ESHAPE outside its
-// shapes, SWAMP_EWORKSPACE without its scratch, nothing launched.
+// The fused GEMM of Q6_K weights (gemm_q6k.hip), with or without scratch for
+// its partial sums; SWAMP_EWORKSPACE, nothing launched, for the shapes it does
+// not take, which only the dequantize-once route's scratch can run.
 size_t swamp_gemm_q6k_scratch_bytes(int m, int n_rows, int n_cols);
 int swamp_launch_gemm_q6k(const void *d_w, const void *d_x, float *d_y, int m, int n_rows,
                           int n_cols, swamp::Scratch &sc, hipStream_t s);
