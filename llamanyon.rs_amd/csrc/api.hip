@@ -21,8 +21,9 @@ namespace swamp {
 // shared by every call of that entry point on that device.  Host code uses
 // it only through the address hipGetSymbolAddress returns for the device
 // (g_scratch), never through its name.
-constexpr size_t kNoAllocScratchBytes = size_t(32) << 20;
-static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
+// Its size is part of the interface; the GEMM plan (dispatch.hpp) keeps calls
+// within it.
+static __device__ __align__(256) uint8_t scratch[SWAMP_NOALLOC_SCRATCH_BYTES];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -427,13 +428,13 @@ int swamp_qgemv_batched_noalloc(uint32_t dtype, const void *d_w, size_t w_len, c
     return accumulate ? SWAMP_OK : fill_zero(d_y, size_t(n_tok) * size_t(n_rows), s);
   const int acc = accumulate ? 1 : 0;
   const size_t need =
-      swamp_batched_scratch_bytes(dtype, n_tok, n_rows, n_cols, acc, kNoAllocScratchBytes);
-  if (need > kNoAllocScratchBytes) return SWAMP_EWORKSPACE;
+      swamp_batched_scratch_bytes(dtype, n_tok, n_rows, n_cols, acc, SWAMP_NOALLOC_SCRATCH_BYTES);
+  if (need > SWAMP_NOALLOC_SCRATCH_BYTES) return SWAMP_EWORKSPACE;
   Scratch sc;
   if (need) {
     if (!g_scratch[dev]) return SWAMP_EWORKSPACE;
     sc.base = static_cast<uint8_t *>(g_scratch[dev]);
-    sc.cap = kNoAllocScratchBytes;
+    sc.cap = SWAMP_NOALLOC_SCRATCH_BYTES;
   }
   return swamp_launch_gemv_batched(dtype, d_w, d_x, d_y, n_tok, n_rows, n_cols, acc, sc, s);
 }
