@@ -157,3 +157,16 @@ def test_q6k_gemm_takes_the_faster_route(rules, m, rows, cols, fused, once):
         assert once <= 1.03 * fused
     else:
         assert fused <= 1.03 * once
+
+
+@pytest.mark.parametrize("dt", [Q4_0, Q8_0, Q4_K, Q6_K])
+def test_gemm_split_shapes_reach_every_part_size(rules, dt):
+    """What test_gpu_gemm_split.py runs on the GPU covers whole tiles, halves and
+    quarters (Q6_K has none) in several K pieces, and a part size unsplit."""
+    import test_gpu_gemm_split
+    plans = [rules.plan(dt, *shape) for shape in test_gpu_gemm_split.SHAPES]
+    assert all(p[0] == SPLIT for p in plans)
+    split = {p[1] for p in plans if p[2] > 1}
+    assert split == ({1, 2} if dt == Q6_K else {1, 2, 4})
+    assert any(p[2] == 1 for p in plans) and any(p[2] == 8 for p in plans)
+    assert not rules.dequantize_once(Q6_K, 777, 4096, 14336)
