@@ -170,3 +170,40 @@ def test_gemm_split_shapes_reach_every_part_size(rules, dt):
     assert split == ({1, 2} if dt == Q6_K else {1, 2, 4})
     assert any(p[2] == 1 for p in plans) and any(p[2] == 8 for p in plans)
     assert not rules.dequantize_once(Q6_K, 777, 4096, 14336)
+
+def plain_split_bytes(dt, m, rows, cols):
+    """Scratch of the simplest split: whole tiles in as many K pieces as the CUs
+    hold or halves in at most 4, by 2.0 and 1.3 us a K step and 6 TB/s for the
+    partial sums.  A plan takes no more than this or than the allocation-free
+    entry point's scratch leaves beside the bf16 x."""
+    steps, tiles = cols // 64, -(-m // 256) * -(-rows // 256)
+
+    def piece(n):
+        k = -(-steps // n)
+        return -(-k // 4) * 4 if dt in (Q4_K, Q6_K) else k
+
+    def us(step, n):
+        return piece(n) * step + ((2 * n + 1) * m * rows * 4 / 6e6 if n > 1 else 0)
+
+    whole = min(CUS // tiles, 8, steps // 8)
+    half = max(1, min(CUS // (2 * tiles), 4, steps // 8)) if 4 * tiles <= CUS else 1
+    pieces = -(-steps // piece(whole if whole >= 2 and us(2.0, whole) < us(1.3, half) else half))
+    return pieces * m * rows * 4 if pieces > 1 else 0
+
+
+@pytest.mark.parametrize("dt", [Q4_0, Q8_0, Q4_K])
+def test_calls_of_the_fixed_scratch_keep_fitting(rules, dt):
+    """swamp_qgemv_batched_noalloc refuses a call whose bf16 x and partial sums
+    exceed its 32 MiB: every shape that fits with the simplest split fits."""
+    limit, pad, near = 32 << 20, lambda b: -(-b // 256) * 256, 0
+    for m in [*range(65, 520, 13), *range(520, 2049, 61)]:
+        for rows in (130, 1000, 1024, 2048, 2560, 3000, 4096, 5120, 6144, 8192, 11008, 14336, 28672):
+            if 2 * -(-m // 256) * -(-rows // 256) > CUS:
+                continue
+            for cols in (512, 1024, 2048, 4096, 5120, 8192, 14336, 28672):
+                xb = pad(m * cols * 2)
+                before = xb + pad(plain_split_bytes(dt, m, rows, cols))
+                now = xb + pad(rules.plan(dt, m, rows, cols)[4])
+                assert now <= max(limit, before), (m, rows, cols)
+                near += 0.8 * limit < now <= limit
+    assert near > 50, near
