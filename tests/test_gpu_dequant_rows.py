@@ -36,3 +36,33 @@ def test_dequant_edges(pkg, orc, dtype, offset):
         nan = np.isnan(want)
         assert np.array_equal(np.isnan(got), nan)
         assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [Q4_0, Q8_0, Q4_K, Q6_K])
+def test_dequant_every_scale_bit_for_bit(pkg, orc, dtype):
+    """A block for each of the 65536 halves as its scale: the lane-contiguous
+    kernel (16-byte aligned output) and the element-store one give the same bits,
+    NaN payloads included, and the oracle's values."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    pkg.init()
+    bs, ts = BLOCK[dtype]
+    raw = np.random.default_rng(dtype).integers(0, 256, (65536, ts), dtype=np.uint8)
+    at = 208 if dtype == Q6_K else 0
+    raw[:, at:at + 2] = np.arange(65536, dtype=np.uint16).view(np.uint8).reshape(-1, 2)
+    raw, n = raw.reshape(-1), 65536 * bs
+    d_raw = torch.from_numpy(raw).cuda()
+    out = []
+    for offset in (0, 1):
+        print("[gpu case] dequant every scale", dtype, offset, flush=True)
+        d_y = torch.empty(n + 4, dtype=torch.float32, device="cuda")
+        pkg.qdequant(dtype, d_raw.data_ptr(), raw.size, d_y.data_ptr() + 4 * offset, n,
+                     torch.cuda.current_stream().cuda_stream)
+        out.append(d_y[offset:offset + n].cpu().numpy())
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+    ref = orc.dequantize(dtype, raw, n)
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(out[0]), nan)
+    assert np.array_equal(out[0][~nan].view(np.uint32), ref[~nan].view(np.uint32))
+
