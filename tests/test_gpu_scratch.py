@@ -59,8 +59,8 @@ def test_workspace_queries(pkg, torch_dev):
     assert L.swamp_qgemm_workspace(Q4_0, BF16, 512, 28672, 4096) == 0
     # full rounds plus a last round of half tiles: no split either
     assert L.swamp_qgemm_workspace(Q4_0, BF16, 2048, 28672, 4096) == 0
-    # between half a round and one round of full tiles at 2048 tokens, and Q6_K:
-    # the dequantize-once route (a bf16 weight chunk)
+    # between half a round and one round of full tiles at 2048 tokens, and Q6_K
+    # of at most 64 tokens: the dequantize-once route (a bf16 weight chunk)
     assert L.swamp_qgemm_workspace(Q4_0, BF16, 2048, 6144, 4096) >= 6144 * 4096 * 2
     assert L.swamp_qgemm_workspace(Q6_K, BF16, 64, 512, 4096) >= 512 * 4096 * 2
     # small batch: K groups on a short matrix (also with token groups, 40
@@ -106,7 +106,8 @@ def test_bench_route_labels_match_library(pkg, torch_dev, monkeypatch):
         assert label.startswith("dequantize-once") == (ws_default == ws_dq), (dt, m, rows, k, label)
         checked += 1
     assert checked >= 6, checked
-    # Q6_K always takes the dequantize-once route
+    # Q6_K reports its dequantized weights on either route, so the rule itself is
+    # compared with the labels instead, without a GPU (test_dispatch_rules.py)
     assert bench.gemm_route(torch, True, 64, 512, 4096, "bf16").startswith("dequantize-once")
 
 
