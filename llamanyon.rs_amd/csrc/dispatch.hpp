@@ -163,8 +163,31 @@ inline bool gemm_dequantize_once(uint32_t dtype, int m, int n_rows, int n_cols, 
   return 2 * tiles > cus && tiles < cus;
 }
 
-// Rows of a 16-row tile of the small-batch kernels.
-constexpr int kBatchTileRows = 16;
+// Rows of a tile of the small-batch kernels, and of a workgroup of 16 tiles.
+constexpr int kBatchTileRows = 16, kBatchGroupRows = 256;
+
+// Whether a small-batch pass splits K over workgroups (each stages a range of x;
+// the partial sums go to scratch and a second kernel adds them), instead of
+// staging all of x into every workgroup in K phases.  It takes at most half the
+// CUs in row groups, and activations worth splitting: from 16384 values, but not
+// where a pass of phases is short.  Timed on 8164 shapes; us, phases / K groups:
+//  * up to 1024 weights, two phases at most: 17 x 6144 x 1024 Q8_0 8.1 / 9.4, 32 x
+//    4096 x 1024 Q4_0 7.9 / 8.9, 63 x 14337 x 1024 12.2 / 18.9; only 33 tokens
+//    and more on few rows gain (64 x 4096 x 1024 11.1 / 10.9);
+//  * up to 2048 weights and 32 tokens: many rows leave only 4 or 5 groups (32 x
+//    12288 x 2048 Q4_K 12.4 / 13.3, 17 x 12288 x 1536 Q4_0 10.2 / 10.5), and at
+//    most 16 tokens stage quickly (16 x 4096 x 2048 Q4_K 7.3 / 8.1, 16 x 2048 x
+//    2048 Q4_0 6.9 / 8.0; but 16 x 4096 x 1536 Q4_K, no whole number of the phases'
+//    granules, 8.3 / 7.8, 16 x 4096 x 1792 8.5 / 7.8);
+//  * beyond, groups gain: 16 x 4096 x 4096 Q4_K 10.0 / 8.8, 32 x 4096 x 2048 Q6_K
+//    12.7 / 11.9, 48 x 1024 x 4096 Q4_0 24.7 / 11.2.
+inline bool small_batch_k_groups(int n_tok, int n_rows, int n_cols, int cus) {
+  const int groups = (n_rows + kBatchGroupRows - 1) / kBatchGroupRows;
+  if (2 * groups > cus || long(n_tok) * n_cols < 16384) return false;
+  if (n_cols <= 1024) return n_tok > 32 && 16 * groups <= cus;
+  if (n_cols <= 2048 && n_tok <= 32) return 32 * groups <= 5 * cus && (n_tok > 16 || n_cols % 1024 != 0);
+  return true;
+}
 
 // Small-batch passes that take gemv_xs_kernel, which loads each wave's share of
 // x into registers, instead of gemv_batched_kernel, which stages x through LDS.

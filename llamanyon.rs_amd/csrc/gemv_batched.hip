@@ -48,6 +48,7 @@ typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kWaves = 16;      // waves per workgroup, one workgroup per CU
+static_assert(kWaves * swamp::kBatchTileRows == swamp::kBatchGroupRows, "a wave per tile");
 constexpr int kThreads = kWaves * 64;
 constexpr int kTok = 64;        // tokens per pass: up to 4 groups of 16 (MFMA M)
 constexpr int kRowsTile = swamp::kBatchTileRows;  // rows per tile (MFMA N)
@@ -922,17 +923,14 @@ int launch_geo_r(Args a, int lwk, int nkg, hipStream_t s) {
 }
 
 // K-group plan of a pass: with one wave per tile (Wk = 1) a workgroup
-// covers 16 tiles; when those tile groups fill at most half the CUs and the
-// pass's activations are not small (n_tok * K >= 16384 fp32, which the
-// K-phase form would stage whole into every workgroup), the row's items are
-// split over workgroups instead, each staging only its range: as many
+// covers 16 tiles; where small_batch_k_groups says so the row's items are
+// split over workgroups instead, each staging only its range of x: as many
 // groups as fill the CUs (at least 4), each a multiple of the chunk granule
 // q (8 items, or 4 when that fills more CUs) and within the LDS.  nkg = 1:
 // no split.
 struct KgPlan {
   int nkg, q;
 };
-constexpr long kKgMinX = 16384;  // n_tok * K from which K groups pay (measured)
 constexpr int kKgMin = 4;        // fewer groups do not pay for the reduction (measured)
 KgPlan kg_plan(int n_tok, int n_rows, int n_cols, int tok) {
   static const int forced = [] {  // tuning override: SWAMP_BATCHED_NKG (1 = off)
@@ -941,10 +939,10 @@ KgPlan kg_plan(int n_tok, int n_rows, int n_cols, int tok) {
   }();
   const int ipr = (n_cols + 63) / 64;
   const int cus = swamp::device_info().num_cus;
-  const int n_tg0 = ((n_rows + kRowsTile - 1) / kRowsTile + kWaves - 1) / kWaves;
+  const int n_tg0 = (n_rows + swamp::kBatchGroupRows - 1) / swamp::kBatchGroupRows;
   const int xcap_items = kXLdsMax / ((tok + 1) * 8 * 16);
   if (forced == 1) return {1, 8};
-  if (forced <= 0 && (2 * n_tg0 > cus || long(n_tok) * n_cols < kKgMinX)) return {1, 8};
+  if (forced <= 0 && !swamp::small_batch_k_groups(n_tok, n_rows, n_cols, cus)) return {1, 8};
   KgPlan best{1, 8};
   for (int q : {8, 4}) {
     const int xcap = xcap_items / q * q;

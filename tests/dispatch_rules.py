@@ -24,6 +24,9 @@ int dequantize_once(unsigned dt, int m, int rows, int cols, int cus) {
 int in_registers(unsigned dt, int n, int rows, int cols, int cus) {
   return swamp::small_batch_in_registers(dt, n, rows, cols, cus);
 }
+int k_groups(int n, int rows, int cols, int cus) {
+  return swamp::small_batch_k_groups(n, rows, cols, cus);
+}
 int product_staged(unsigned dt, int rows, int cols, int add, int cus) {
   return swamp::swiglu_product_staged(dt, rows, cols, add != 0, cus);
 }
@@ -55,3 +58,6 @@ class Rules:
 
     def product_staged(self, dt, rows, cols, add=False, cus=CUS):
         return bool(self.lib.product_staged(dt, rows, cols, int(add), cus))
+
+    def k_groups(self, n, rows, cols, cus=CUS):
+        return bool(self.lib.k_groups(n, rows, cols, cus))

@@ -207,3 +207,24 @@ def test_calls_of_the_fixed_scratch_keep_fitting(rules, dt):
                 assert now <= max(limit, before), (m, rows, cols)
                 near += 0.8 * limit < now <= limit
     assert near > 50, near
+
+
+# (tokens, rows, weights per row, us in K phases, us in K groups), the format each
+# was measured with beside it
+K_GROUPS = [
+    (32, 4096, 1024, 7.91, 8.94), (25, 14337, 1024, 8.14, 12.04), (63, 14337, 1024, 12.22, 18.93),
+    (64, 4096, 1024, 11.11, 10.87), (16, 2048, 2048, 6.94, 7.95), (50, 16384, 2048, 18.56, 18.51),
+    (17, 12288, 1536, 10.23, 10.50), (8, 4096, 6144, 11.69, 10.48), (48, 1024, 4096, 24.73, 11.17),  # Q4_0
+    (17, 6144, 1024, 8.05, 9.37), (32, 14337, 2048, 15.74, 17.55),  # Q8_0
+    (16, 4096, 2048, 7.26, 8.13), (16, 4096, 1536, 8.28, 7.77), (16, 12288, 1536, 8.88, 9.98),
+    (16, 4096, 1792, 8.52, 7.80),
+    (32, 12288, 2048, 12.43, 13.27), (32, 4096, 2048, 10.14, 9.70), (16, 4096, 4096, 9.99, 8.78),  # Q4_K
+    (25, 6144, 1024, 9.88, 11.64), (32, 4096, 2048, 12.72, 11.91), (32, 4096, 1536, 12.99, 11.62)]  # Q6_K
+
+
+@pytest.mark.parametrize("n,rows,cols,phases,groups", K_GROUPS)
+def test_small_batch_splits_k_where_it_is_faster(rules, n, rows, cols, phases, groups):
+    if rules.k_groups(n, rows, cols):
+        assert groups <= 1.03 * phases
+    else:
+        assert phases <= 1.03 * groups
