@@ -196,12 +196,14 @@ inline bool small_batch_k_groups(int n_tok, int n_rows, int n_cols, int cus) {
 // 16 tokens x 256 to 32768 rows x 256 to 32768 weights; us, staged / registers:
 //  * One tile per workgroup (rows <= 16 x the CUs): 16 waves take up to 4096
 //    weights in one pass (rows of 14336 lose, 14.5 / 22.0).  Q6_K gains up to 32768 x
-//    values: 1024 x 4096 at 5 tokens 10.5 / 8.4, 4096 x 2048 at 16 10.3 / 8.9.
-//    Q8_0 4096 x 2048 at 14 9.6 / 9.0, but 4096 x 2560 at 12 8.7 / 9.1; Q4_0
-//    4096 x 2048 at 12 8.1 / 7.6, but 4096 x 4096 at 8 8.2 / 8.8.
+//    values: 1024 x 4096 at 5 tokens 10.4 / 8.3, 4096 x 2048 at 16 9.9 / 8.9.
+//    Q8_0 4096 x 4096 at 5 9.9 / 8.6, but 4096 x 2560 at 12 8.8 / 9.1; Q4_0 4096 x
+//    4096 at 5 8.0 / 7.6, at 8 8.1 / 9.0.  Rows of 2048 weights are one phase of
+//    the staged kernel: Q8_0 4096 x 2048 at 8 8.2 / 7.6, at 14 8.4 / 8.9, Q4_0 at 6
+//    6.8 / 6.5, at 12 7.1 / 7.5.
 //  * Q4_K's scale unpacking makes the line fall faster than the token count
-//    rises: 4096 x 4096 at 5 8.0 / 7.5, at 6 8.1 / 8.4, at 8 8.1 / 10.0; 4096 x
-//    2048 at 8 7.8 / 7.7, at 16 8.6 / 11.8.  Rows that are not whole 1024-weight
+//    rises: 4096 x 4096 at 5 7.9 / 7.5, at 6 8.0 / 8.4, at 8 8.1 / 10.1; 4096 x
+//    2048 at 8 7.1 / 7.7, at 16 7.5 / 11.7.  Rows that are not whole 1024-weight
 //    granules of the staged kernel leave more room: 4096 x 1280 at 12 8.1 / 7.7.
 //  * Rows of 256 weights gain nothing (5.1 / 5.3).
 //  * More rows take 2 to 8 tiles per workgroup, whose 8 waves are all busy when
@@ -217,20 +219,23 @@ inline bool small_batch_in_registers(uint32_t dtype, int n_tok, int n_rows, int 
   const int n_tiles = (n_rows + kBatchTileRows - 1) / kBatchTileRows;
   const int nt = (n_tiles + cus - 1) / cus;  // tiles per workgroup
   const long nx = long(n_tok) * n_cols;
-  const bool nibbles = dtype == SWAMP_Q4_0 || dtype == SWAMP_Q4_K;
+  const bool nibbles = dtype == SWAMP_Q4_0 || dtype == SWAMP_Q4_K, q8 = dtype == SWAMP_Q8_0;
   if (n_tok > 16 || n_cols % 256 != 0 || n_cols < 512) return false;
   if (nt <= 1) {
-    if (n_cols > 4096) return false;
+    if (n_cols > 4096 || (n_cols == 2048 && n_tok > (nibbles ? 6 : q8 ? 9 : 16))) return false;
     if (dtype == SWAMP_Q4_K)
-      return nx <= 21504 && nx * n_tok <= (n_cols % 1024 ? 196608 : 131072);
-    return nx <= (dtype == SWAMP_Q6_K ? 32768 : dtype == SWAMP_Q8_0 ? 28672 : 27648);
+      return nx <= 21504 && nx * n_tok <= (n_cols % 1024 ? 196608 : n_cols > 1024 ? 131072 : 98304);
+    return nx <= (q8 ? 28672 : nibbles ? 27648 : 32768);
   }
   if (nt > 8 || n_cols % 2048 != 0) return false;
-  if (nibbles)
-    return n_cols <= (nt <= 4 ? 4096 : 2048) && nt != 5 && nt != 6 &&
-           n_tok >= (nt <= 3 ? 2 : 3) && nx <= (nt == 3 || nt == 4 ? 32768 : 28672);
-  if (n_cols <= 4096) return nx <= (nt >= 3 ? 57344 : 32768);
-  return n_cols <= 8192 && nt >= 4 && nt <= (dtype == SWAMP_Q8_0 ? 5 : 4) && nx <= 32768;
+  if (nibbles) {
+    if (n_tok < (nt <= 3 ? 2 : 3) || nt == 5 || nt == 6) return false;
+    if (n_cols == 2048) return n_tok <= (nt == 2 ? 9 : 12);
+    return n_cols == 4096 && nt <= 4 && nx <= (nt == 2 ? 28672 : 32768);
+  }
+  if (n_cols == 2048) return n_tok <= (q8 && nt == 2 ? 13 : 16);
+  if (n_cols == 4096) return nx <= (nt >= 3 ? 57344 : 32768);
+  return n_cols <= 8192 && nt >= 4 && nt <= (q8 ? 5 : 4) && nx <= 32768;
 }
 
 // Whether the decode GEMV behind SwiGLU forms silu(gate) * up once per

@@ -41,28 +41,32 @@ def test_bench_route_labels_follow_the_rule(rules, bench):
 # (dtype, tokens, rows, weights per row, us staged, us in registers), measured on
 # an MI355X over rotating weights
 SMALL_BATCH = [
-    (Q4_0, 1, 4096, 256, 5.10, 5.25), (Q4_0, 5, 4096, 4096, 7.97, 7.55),
-    (Q4_0, 8, 4096, 4096, 8.16, 8.81), (Q4_0, 12, 4096, 2048, 8.07, 7.56),
-    (Q4_0, 8, 14336, 2048, 10.86, 9.50), (Q4_0, 5, 14336, 4096, 15.59, 14.06),
-    (Q4_0, 3, 5120, 8192, 12.30, 15.51), (Q4_0, 1, 16384, 4096, 13.85, 14.56),
-    (Q4_0, 12, 28672, 2048, 15.45, 14.41), (Q4_0, 1, 5120, 28672, 24.97, 38.96),
-    (Q8_0, 5, 4096, 4096, 9.92, 8.68), (Q8_0, 14, 4096, 2048, 9.58, 9.00),
-    (Q8_0, 12, 4096, 2560, 8.72, 9.12), (Q8_0, 5, 14336, 4096, 22.42, 19.67),
-    (Q8_0, 14, 14336, 4096, 24.41, 22.79), (Q8_0, 4, 5120, 8192, 17.69, 20.71),
-    (Q8_0, 1, 5120, 28672, 38.38, 55.86), (Q8_0, 3, 5120, 10240, 20.48, 24.49),
-    (Q4_K, 3, 4096, 4096, 7.71, 7.12), (Q4_K, 5, 4096, 4096, 7.96, 7.50),
-    (Q4_K, 5, 1024, 4096, 7.89, 7.31), (Q4_K, 6, 4096, 4096, 8.05, 8.40),
-    (Q4_K, 8, 4096, 4096, 8.11, 10.04), (Q4_K, 9, 4096, 3584, 7.93, 9.34),
-    (Q4_K, 10, 4096, 2560, 7.76, 9.08), (Q4_K, 12, 4096, 2560, 7.85, 10.17),
-    (Q4_K, 12, 4096, 1280, 8.10, 7.66), (Q4_K, 16, 4096, 768, 7.56, 6.94),
-    (Q4_K, 16, 4096, 2048, 8.61, 11.78), (Q4_K, 16, 1024, 2048, 8.16, 9.33),
-    (Q4_K, 5, 14336, 4096, 15.97, 14.38), (Q4_K, 1, 16384, 4096, 13.66, 14.48),
-    (Q4_K, 4, 5120, 8192, 12.69, 16.16), (Q4_K, 2, 5120, 14336, 16.65, 23.44),
-    (Q4_K, 16, 20480, 2048, 13.37, 14.79), (Q4_K, 8, 28672, 2048, 14.86, 13.79),
-    (Q6_K, 5, 1024, 4096, 10.45, 8.36), (Q6_K, 8, 4096, 4096, 10.55, 9.63),
-    (Q6_K, 16, 4096, 2048, 10.30, 8.88), (Q6_K, 4, 5120, 8192, 18.00, 22.28),
-    (Q6_K, 5, 14336, 6144, 27.57, 25.24), (Q6_K, 3, 5120, 6144, 14.03, 16.42),
-    (Q6_K, 5, 28672, 4096, 31.09, 29.57)]
+    (Q4_0, 1, 4096, 256, 5.15, 5.29), (Q4_0, 5, 4096, 4096, 7.99, 7.59),
+    (Q4_0, 8, 4096, 4096, 8.12, 9.01), (Q4_0, 12, 4096, 2048, 7.13, 7.51),
+    (Q4_0, 8, 14336, 2048, 9.64, 9.38), (Q4_0, 5, 14336, 4096, 15.72, 14.06),
+    (Q4_0, 3, 5120, 8192, 12.30, 15.14), (Q4_0, 1, 16384, 4096, 13.70, 14.46),
+    (Q4_0, 12, 28672, 2048, 15.15, 14.19), (Q4_0, 1, 5120, 28672, 24.97, 38.96),
+    (Q4_0, 6, 4096, 2048, 6.76, 6.46), (Q4_0, 9, 2048, 2048, 6.97, 6.77),
+    (Q4_0, 12, 14336, 2048, 10.28, 10.25), (Q8_0, 5, 4096, 4096, 9.86, 8.62),
+    (Q8_0, 14, 4096, 2048, 8.35, 8.94), (Q8_0, 12, 4096, 2560, 8.77, 9.14),
+    (Q8_0, 5, 14336, 4096, 22.37, 19.74), (Q8_0, 14, 14336, 4096, 24.24, 22.49),
+    (Q8_0, 4, 5120, 8192, 17.38, 20.60), (Q8_0, 1, 5120, 28672, 38.38, 55.86),
+    (Q8_0, 3, 5120, 10240, 20.48, 24.49), (Q8_0, 8, 4096, 2048, 8.16, 7.57),
+    (Q8_0, 16, 2560, 2048, 8.16, 9.23), (Q4_K, 3, 4096, 4096, 7.70, 7.14),
+    (Q4_K, 5, 4096, 4096, 7.91, 7.45), (Q4_K, 5, 1024, 4096, 7.88, 7.35),
+    (Q4_K, 6, 4096, 4096, 7.97, 8.38), (Q4_K, 8, 4096, 4096, 8.10, 10.08),
+    (Q4_K, 9, 4096, 3584, 7.94, 9.36), (Q4_K, 10, 4096, 2560, 7.76, 9.02),
+    (Q4_K, 12, 4096, 2560, 7.87, 10.23), (Q4_K, 12, 4096, 1280, 8.12, 7.72),
+    (Q4_K, 16, 4096, 768, 7.67, 7.08), (Q4_K, 16, 4096, 2048, 7.53, 11.65),
+    (Q4_K, 16, 1024, 2048, 6.82, 8.62), (Q4_K, 5, 14336, 4096, 15.73, 14.43),
+    (Q4_K, 1, 16384, 4096, 13.60, 14.51), (Q4_K, 4, 5120, 8192, 12.60, 16.14),
+    (Q4_K, 2, 5120, 14336, 16.65, 23.44), (Q4_K, 16, 20480, 2048, 12.94, 14.90),
+    (Q4_K, 8, 28672, 2048, 14.77, 13.76), (Q4_K, 8, 4096, 2048, 7.13, 7.66),
+    (Q4_K, 14, 5120, 2048, 7.71, 8.52), (Q4_K, 11, 4096, 1024, 6.56, 6.99),
+    (Q6_K, 5, 1024, 4096, 10.36, 8.34),
+    (Q6_K, 8, 4096, 4096, 10.49, 9.66), (Q6_K, 16, 4096, 2048, 9.87, 8.86),
+    (Q6_K, 4, 5120, 8192, 18.06, 21.80), (Q6_K, 5, 14336, 6144, 27.27, 24.70),
+    (Q6_K, 3, 5120, 6144, 13.95, 16.19), (Q6_K, 5, 28672, 4096, 31.03, 29.60)]
 
 
 @pytest.mark.parametrize("dt,n,rows,cols,staged,registers", SMALL_BATCH)
