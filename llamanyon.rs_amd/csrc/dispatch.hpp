@@ -185,7 +185,8 @@ inline bool small_batch_k_groups(int n_tok, int n_rows, int n_cols, int cus) {
   const int groups = (n_rows + kBatchGroupRows - 1) / kBatchGroupRows;
   if (2 * groups > cus || long(n_tok) * n_cols < 16384) return false;
   if (n_cols <= 1024) return n_tok > 32 && 16 * groups <= cus;
-  if (n_cols <= 2048 && n_tok <= 32) return 32 * groups <= 5 * cus && (n_tok > 16 || n_cols % 1024 != 0);
+  if (n_cols <= 2048 && n_tok <= 32)
+    return 32 * groups <= 5 * cus && (n_tok > 16 || n_cols % 1024 != 0);
   return true;
 }
 
@@ -204,7 +205,8 @@ inline bool small_batch_k_groups(int n_tok, int n_rows, int n_cols, int cus) {
 //  * Q4_K's scale unpacking makes the line fall faster than the token count
 //    rises: 4096 x 4096 at 5 7.9 / 7.5, at 6 8.0 / 8.4, at 8 8.1 / 10.1; 4096 x
 //    2048 at 8 7.1 / 7.7, at 16 7.5 / 11.7.  Rows that are not whole 1024-weight
-//    granules of the staged kernel leave more room: 4096 x 1280 at 12 8.1 / 7.7.
+//    granules of the staged kernel leave more room, most on few tiles: 4096 x
+//    1280 at 12 8.1 / 7.7, 512 x 1280 at 14 7.2 / 6.2.
 //  * Rows of 256 weights gain nothing (5.1 / 5.3).
 //  * More rows take 2 to 8 tiles per workgroup, whose 8 waves are all busy when
 //    the row is whole 2048-weight passes; each pass beyond the second costs
@@ -223,8 +225,11 @@ inline bool small_batch_in_registers(uint32_t dtype, int n_tok, int n_rows, int 
   if (n_tok > 16 || n_cols % 256 != 0 || n_cols < 512) return false;
   if (nt <= 1) {
     if (n_cols > 4096 || (n_cols == 2048 && n_tok > (nibbles ? 6 : q8 ? 9 : 16))) return false;
-    if (dtype == SWAMP_Q4_K)
-      return nx <= 21504 && nx * n_tok <= (n_cols % 1024 ? 196608 : n_cols > 1024 ? 131072 : 98304);
+    if (dtype == SWAMP_Q4_K) {
+      if (n_cols % 1024 == 0) return nx * n_tok <= (n_cols > 1024 ? 131072 : 98304);
+      if (n_cols < 2048 && 4 * n_tiles <= cus) return true;
+      return nx <= 21504 && nx * n_tok <= (8 * n_tiles <= 5 * cus ? 262144 : 196608);
+    }
     return nx <= (q8 ? 28672 : nibbles ? 27648 : 32768);
   }
   if (nt > 8 || n_cols % 2048 != 0) return false;

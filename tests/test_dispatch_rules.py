@@ -63,6 +63,8 @@ SMALL_BATCH = [
     (Q4_K, 2, 5120, 14336, 16.65, 23.44), (Q4_K, 16, 20480, 2048, 12.94, 14.90),
     (Q4_K, 8, 28672, 2048, 14.77, 13.76), (Q4_K, 8, 4096, 2048, 7.13, 7.66),
     (Q4_K, 14, 5120, 2048, 7.71, 8.52), (Q4_K, 11, 4096, 1024, 6.56, 6.99),
+    (Q4_K, 14, 512, 1280, 7.25, 6.18), (Q4_K, 13, 512, 1536, 7.68, 6.34),
+    (Q4_K, 16, 4096, 1280, 7.75, 8.72),
     (Q6_K, 5, 1024, 4096, 10.36, 8.34),
     (Q6_K, 8, 4096, 4096, 10.49, 9.66), (Q6_K, 16, 4096, 2048, 9.87, 8.86),
     (Q6_K, 4, 5120, 8192, 18.06, 21.80), (Q6_K, 5, 14336, 6144, 27.27, 24.70),
@@ -150,8 +152,9 @@ Q6K_ROUTES = [
     (512, 28672, 4096, 148.6, 183.4), (512, 128256, 4096, 630.0, 769.2),
     (520, 6144, 14336, 167.9, 265.4), (700, 7168, 10240, 153.0, 190.6),
     (777, 2048, 28672, 150.2, 164.5), (777, 4096, 14336, 143.2, 157.9),
-    (1000, 2048, 8192, 70.4, 61.0), (1000, 6144, 4096, 102.2, 74.6), (1300, 4096, 8192, 140.6, 117.1),
-    (1300, 6144, 14336, 394.4, 338.7), (1700, 1024, 8192, 66.2, 55.9), (1700, 1024, 28672, 149.5, 161.3),
+    (1000, 2048, 8192, 70.4, 61.0), (1000, 6144, 4096, 102.2, 74.6),
+    (1300, 4096, 8192, 140.6, 117.1), (1300, 6144, 14336, 394.4, 338.7),
+    (1700, 1024, 8192, 66.2, 55.9), (1700, 1024, 28672, 149.5, 161.3),
     (2048, 3000, 8192, 145.1, 121.5), (2048, 4096, 8192, 172.7, 152.6)]
 
 
@@ -201,7 +204,8 @@ def test_calls_of_the_fixed_scratch_keep_fitting(rules, dt):
     exceed its 32 MiB: every shape that fits with the simplest split fits."""
     limit, pad, near = 32 << 20, lambda b: -(-b // 256) * 256, 0
     for m in [*range(65, 520, 13), *range(520, 2049, 61)]:
-        for rows in (130, 1000, 1024, 2048, 2560, 3000, 4096, 5120, 6144, 8192, 11008, 14336, 28672):
+        for rows in (130, 1000, 1024, 2048, 2560, 3000, 4096, 5120, 6144, 8192, 11008, 14336,
+                     28672):
             if 2 * -(-m // 256) * -(-rows // 256) > CUS:
                 continue
             for cols in (512, 1024, 2048, 4096, 5120, 8192, 14336, 28672):
@@ -213,17 +217,20 @@ def test_calls_of_the_fixed_scratch_keep_fitting(rules, dt):
     assert near > 50, near
 
 
-# (tokens, rows, weights per row, us in K phases, us in K groups), the format each
-# was measured with beside it
+# (tokens, rows, weights per row, us in K phases, us in K groups)
 K_GROUPS = [
+    # Q4_0
     (32, 4096, 1024, 7.91, 8.94), (25, 14337, 1024, 8.14, 12.04), (63, 14337, 1024, 12.22, 18.93),
     (64, 4096, 1024, 11.11, 10.87), (16, 2048, 2048, 6.94, 7.95), (50, 16384, 2048, 18.56, 18.51),
-    (17, 12288, 1536, 10.23, 10.50), (8, 4096, 6144, 11.69, 10.48), (48, 1024, 4096, 24.73, 11.17),  # Q4_0
-    (17, 6144, 1024, 8.05, 9.37), (32, 14337, 2048, 15.74, 17.55),  # Q8_0
+    (17, 12288, 1536, 10.23, 10.50), (8, 4096, 6144, 11.69, 10.48), (48, 1024, 4096, 24.73, 11.17),
+    # Q8_0
+    (17, 6144, 1024, 8.05, 9.37), (32, 14337, 2048, 15.74, 17.55),
+    # Q4_K
     (16, 4096, 2048, 7.26, 8.13), (16, 4096, 1536, 8.28, 7.77), (16, 12288, 1536, 8.88, 9.98),
-    (16, 4096, 1792, 8.52, 7.80),
-    (32, 12288, 2048, 12.43, 13.27), (32, 4096, 2048, 10.14, 9.70), (16, 4096, 4096, 9.99, 8.78),  # Q4_K
-    (25, 6144, 1024, 9.88, 11.64), (32, 4096, 2048, 12.72, 11.91), (32, 4096, 1536, 12.99, 11.62)]  # Q6_K
+    (16, 4096, 1792, 8.52, 7.80), (32, 12288, 2048, 12.43, 13.27), (32, 4096, 2048, 10.14, 9.70),
+    (16, 4096, 4096, 9.99, 8.78),
+    # Q6_K
+    (25, 6144, 1024, 9.88, 11.64), (32, 4096, 2048, 12.72, 11.91), (32, 4096, 1536, 12.99, 11.62)]
 
 
 @pytest.mark.parametrize("n,rows,cols,phases,groups", K_GROUPS)
