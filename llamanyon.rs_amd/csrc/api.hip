@@ -1,7 +1,8 @@
 // api.hip -- the C ABI of libswamp_gpu.so (declared in include/swamp_qmm.h).
 //
 // Validation and dispatch only; kernels live in dequant.hip, gemv.hip,
-// gemv_fused.hip, gemv_batched.hip, gemm.hip and gemm_i8.hip.  The error behaviour mirrors the
+// gemv_fused.hip, gemv_batched.hip, gemm.hip and gemm_i8.hip, and the rules
+// that choose between them by size in dispatch.hpp.  The error behaviour mirrors the
 // reference: shape asserts of fused_gemv_q4k (fused_gemv_q4k.rs:66-70) and
 // the bail! of forward_linear (linear.rs:23-25) become negative return
 // codes, checked before anything is launched; the two legacy host-pointer

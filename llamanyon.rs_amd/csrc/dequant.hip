@@ -159,10 +159,12 @@ __global__ void dequant_q6_k_kernel(const uint8_t *__restrict__ raw,
 // wave two steps of 1 KB, whose loads are all issued before the first
 // conversion.  Stores of fp32 are non-temporal: the output is larger than
 // the caches' share and is not read back here.  14336 x 4096 weights, us (one
-// thread per 8 outputs, two 16-byte stores 32 bytes apart / this kernel):
-// fp32 Q4_0 43.4 / 37.4, Q8_0 65.5 / 41.7, Q4_K 44.9 / 37.7, Q6_K 64.5 / 40.1
-// (7.05-7.17 TB/s); bf16 Q6_K 29.7 / 25.4.  One step per wave measured 39-62
-// us, four 38-43; temporal stores 38.5-54.
+// thread per 8 outputs, two 16-byte stores 32 bytes apart / this kernel), 12
+// weight and output buffers of random blocks in turn: fp32 Q4_0 66.6 / 47.8,
+// Q8_0 61.6 / 52.8, Q4_K 67.2 / 53.6, Q6_K 67.8 / 57.3; bf16 Q6_K 41.3 / 35.0;
+// quantized normal weights, 4 buffers in turn: Q4_K 66.6 / 37.5 (7.1 TB/s).  One
+// step per wave measured 51-60 us where two took 46-55, four 48-52; temporal
+// stores are within 2% of these.
 // Values are those of the kernels above: V_CVT_F32_F16 gives the bits of
 // f16_bits_to_f32_exact for all 65536 halves, NaN payloads included.
 constexpr int kSteps = 2;

@@ -33,8 +33,8 @@ constexpr int kGemmTokens = 256, kGemmRows = 256, kGemmK = 64;
 // weights, all formats; it meets those near the best of their shape within 3%
 // rms): 13 us to fill a whole tile's stages and store it, the K steps below
 // while a round is full (0.78 of a step when few tiles are in flight), 5.7 us for
-// the second kernel and its partial sums, written and read, at 2.3 TB/s per
-// piece.  The choice is within 0.5% of the best on average, 16% at worst.  An
+// the second kernel and 3.4 TB/s for its partial sums, written and read.  The
+// choice is within 0.5% of the best on average, 16% at worst.  An
 // estimate from single shapes (2.04 us a step, 2 us for the second kernel) had
 // split where it does not pay and taken halves where whole tiles in two pieces
 // are faster: us, that choice / this one, 256 tokens x 4096 x 1024 Q4_0 19.2 /

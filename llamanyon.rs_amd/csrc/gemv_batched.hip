@@ -1035,8 +1035,9 @@ namespace {
 int pass_len(uint32_t dtype) { return dtype == SWAMP_Q6_K ? 32 : kTok; }
 
 // The GEMM route of a call: more than 64 tokens written over y, on x rounded
-// to bf16 (in scratch).  Q6_K stays on the passes at any count: its GEMM
-// needs a bf16 copy of the weights in scratch, which the passes do not.
+// to bf16 (in scratch).  Q6_K stays on the passes at any count, which is the
+// entry point's contract for it: x rounded to fp16, no scratch that the passes
+// cannot do without.
 bool gemm_route(uint32_t dtype, int n_tok, int n_cols, int accumulate) {
   return dtype != SWAMP_Q6_K && n_tok > kTok && !accumulate && n_cols % 64 == 0 &&
          size_t(n_tok) * size_t(n_cols) * 2 <= size_t(UINT32_MAX);
