@@ -451,7 +451,8 @@ size_t swamp_qgemm_workspace(uint32_t dtype, uint32_t x_type, int m, int n_rows,
   const size_t need = swamp_gemm_scratch_bytes(dtype, x_type, m, n_rows, n_cols);
   // Q6_K prompts of a few tokens run only with their weights dequantized to
   // scratch: what a long prompt reports holds those too
-  if (dtype == SWAMP_Q6_K && x_type == SWAMP_BF16 && m > 0 && n_rows > 0 && n_cols > 0)
+  if (dtype == SWAMP_Q6_K && x_type == SWAMP_BF16 && m > 0 && n_rows > 0 && n_cols > 0 &&
+      n_cols % 64 == 0)
     return std::max(need, swamp_gemm_dq_scratch_bytes(m, n_rows, n_cols));
   return need;
 }

@@ -84,6 +84,11 @@ def test_long_prompt_reservation_runs_short_prompts(pkg, torch_dev):
     replays(torch, stream, calls, lambda c, rep: _equal(torch, c, want[c.m], rep))
 
 
+def test_report_of_shapes_that_are_refused(pkg, torch_dev):
+    for m, rows, cols in [(0, 4, 512), (4, 0, 512), (4, 4, 0), (-1, 4, 512), (4, 4, 100)]:
+        assert report(pkg, m, rows, cols) == 0, (m, rows, cols)
+
+
 def _equal(torch, c, want, rep):
     assert torch.equal(c.y, want), (c.m, c.rows, c.cols, rep)
 
